@@ -10,21 +10,17 @@
 //   embed scatter  the loop of bridge.m:922-928 adds row i of dx0 into the
 //       embedding row of token i, in increasing i.  Atomics would add in an
 //       arbitrary order and change the fp32 sums, so instead:
-//         1. key = clamped token, value = position i, and a stable LSD radix
-//            sort of (key, i) over the key's bits, which keeps equal keys in
-//            increasing i: for up to kSortTile tokens (the reference's
-//            2 x 2048 batch) one block sorts them in LDS (block_sort_kernel),
-//            beyond that one hist/scan/scatter launch triple per 8-bit digit;
-//         2. gather_kernel: the dx0 rows copied in sorted order into a
-//            workspace, so every run of equal keys is contiguous;
-//         3. run_kernel: one 256-lane block per (run of equal keys,
-//            256-column tile) finds the run's end by binary search, loads the
-//            embedding row once, adds the run's rows in sorted (= original)
-//            order and stores it once.  A run of kLongRun rows or more gives
-//            each lane one column and keeps kColRows rows' loads in flight
-//            (the run is a sequential fp32 chain per column, so its time is
-//            load round trips); a shorter run is done by the first wave alone
-//            with 16-byte accesses.
+//         1. the positions sorted by (clamped token, position): up to
+//            kRankTokens tokens (the reference's batch is 2 x 2048) every
+//            position's place is counted directly (rank_sort_kernel); beyond
+//            that a stable LSD radix sort, one hist/scan/scatter launch triple
+//            per 8-bit digit;
+//         2. run_kernel: the rows of each run of equal tokens, read from dx0
+//            by their sorted positions, added in that (= the original) order
+//            to the embedding row, which is loaded and stored once.  A run of
+//            kLongRun rows or more is a sequential fp32 chain per column
+//            whose loads a whole block keeps in flight; a shorter run is one
+//            wave's per 256 columns.
 //       Every element therefore sees the same additions in the same order as
 //       the CPU loop, and the result is bit-identical.
 #include <stdlib.h>
@@ -55,13 +51,29 @@ constexpr uint32_t kBlocksPerSeg = kSeg / (kWave * kPerLane);  // 16
 // every slot: its per-wave tree of squares shows at fewer waves (470.7
 // against 443.0 us at 24 per CU, same box).
 constexpr int kPlanBlocksPerCu = 24;
-constexpr int kTileCols = 256;  // run_kernel: columns per block
-constexpr int kLongRun = 8;     // runs of at least this many rows: one column per lane
-// Rows in flight per lane on a long run.  Measured on MI355X (4096 tokens,
-// d 768): 60 rows with one column per lane run a single 4096-row run in 73 us
-// against 400 us for 32 rows of four columns; more than 60 gain nothing, a
-// wave keeping at most 63 vector loads outstanding.
-constexpr int kColRows = 60;
+constexpr uint32_t kTileCols = 256;  // columns per wave on a short run, and per norm unit
+// run_kernel's shape.  It is bound by latency: a wave's chain is keys, rows,
+// store, and most waves find no run of theirs and leave, so what counts is how
+// many blocks are resident at once.  Measured on MI355X, 4096 Zipf tokens of
+// 768 columns (18.3 us before, plus 8.8 us for a copy of the rows in sorted
+// order): 18.6 us with 16-wave blocks (74 registers, one block per CU), 22.7 us
+// with 4-wave blocks and runs up to 64 rows left to one wave, 9.4-10.1 us as
+// here, in 62 registers.  One token at all 4096 positions: 25 us (73 us).
+constexpr uint32_t kLongRun = 32;  // runs of at least this many rows go to a whole block
+constexpr uint32_t kRowBatch = 8;  // rows in flight per wave on a short run
+constexpr uint32_t kRunWaves = 8;  // waves per block
+constexpr uint32_t kColRows = 48;  // rows in flight per wave on a long run
+// The sort by counting (rank_sort_kernel): positions per wave and block, keys
+// staged per LDS tile, and the most tokens it takes.  The work grows with the
+// square of the batch.  Measured on MI355X against the radix passes (32 us at
+// 12289 tokens, six launches; one block sorting 4096 tokens in LDS 9.7 us):
+// 2.9 us for 64 tokens, 5.3 for 4096, 11.0 for 8192, 19.1 for 12288, about 33
+// for 16384.
+constexpr uint32_t kRankWaves = 8;
+constexpr int kRankPerWave = 2;
+constexpr uint32_t kRankPerBlock = kRankWaves * kRankPerWave;
+constexpr uint32_t kRankTile = 4096;
+constexpr uint32_t kRankTokens = 12288;
 
 struct GradSeg {
   float* dst;
@@ -231,11 +243,10 @@ __global__ __launch_bounds__(kWave) void units_rows_kernel(const float* __restri
 // Equal digits keep their position order, so each pass is stable and the
 // passes from the low bits up (LSD) leave the keys sorted with equal keys in
 // increasing position: the order in which bridge.m:922-928's loop visits a
-// token's rows.  Up to one tile (the reference's 2 x 2048 batch) one block
-// does every pass in LDS (block_sort_kernel); past that each pass is three
-// launches: per-tile digit counts (sort_hist_kernel), their exclusive scan
-// in (digit, tile) order (sort_scan_kernel), and the tile-local rank plus the
-// scanned count as the global destination (sort_scatter_kernel).
+// token's rows.  Each pass is three launches: per-tile digit counts
+// (sort_hist_kernel), their exclusive scan in (digit, tile) order
+// (sort_scan_kernel), and the tile-local rank plus the scanned count as the
+// global destination (sort_scatter_kernel).
 constexpr int kSortThreads = 1024;
 constexpr int kSortWaves = kSortThreads / kWave;                // 16
 constexpr int kSortItems = 4;
@@ -350,51 +361,6 @@ __device__ __forceinline__ void tile_pass(const uint32_t (&dig)[kSortItems],
   __syncthreads();
 }
 
-// Up to kSortTile tokens: one block sorts (key = clamped token, value =
-// position) over bits [0, end_bit) in LDS and writes the first n pairs.
-// Positions past n take the all-ones key: its digit is the largest in every
-// pass and it comes after every real item, so it sorts after them all.
-__global__ __launch_bounds__(kSortThreads) void block_sort_kernel(
-    const uint32_t* __restrict__ tokens, uint32_t n, uint32_t vocab, int end_bit,
-    uint32_t* __restrict__ skeys, uint32_t* __restrict__ svals) {
-  __shared__ uint32_t s_keys[kSortTile], s_vals[kSortTile], s_hist[kHistWords],
-      s_wsum[kSortWaves];
-  const uint32_t lane = __lane_id(), wave = threadIdx.x / kWave;
-  uint32_t k[kSortItems], v[kSortItems], dg[kSortItems], r[kSortItems];
-#pragma unroll
-  for (int j = 0; j < kSortItems; ++j) {
-    const uint32_t p = tile_pos(wave, j, lane);
-    k[j] = p < n ? clamp_token(ld_g<uint32_t>(tokens + p), vocab) : kPadKey;
-    v[j] = p;
-  }
-  for (int shift = 0; shift < end_bit; shift += kRadixBits) {
-#pragma unroll
-    for (int j = 0; j < kSortItems; ++j) dg[j] = (k[j] >> shift) & (kRadix - 1u);
-    tile_pass(dg, r, s_hist, s_wsum);
-#pragma unroll
-    for (int j = 0; j < kSortItems; ++j) {
-      const uint32_t dst = s_hist[hist_at(dg[j], wave)] + r[j];
-      s_keys[dst] = k[j];
-      s_vals[dst] = v[j];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kSortItems; ++j) {
-      const uint32_t p = tile_pos(wave, j, lane);
-      k[j] = s_keys[p];
-      v[j] = s_vals[p];
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < kSortItems; ++j) {
-    const uint32_t p = tile_pos(wave, j, lane);
-    if (p < n) {
-      skeys[p] = k[j];
-      svals[p] = v[j];
-    }
-  }
-}
-
 // counts[d * tiles + tile] = the items of the tile whose key has digit d at
 // this pass: the waves' counters of wave_rank, summed over the waves.
 // from_tokens: the keys are the clamped tokens (first pass).  Positions past
@@ -499,134 +465,342 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(
   }
 }
 
-// Row q of xs = row svals[q] of dx0 (d floats each); one block per row.
-// vec: d % 4 == 0 and dx0 16-byte aligned (xs is 256-byte aligned).
-__global__ __launch_bounds__(kThreads) void gather_kernel(const float* __restrict__ dx0,
-                                                          const uint32_t* __restrict__ svals,
-                                                          uint32_t d, uint32_t vec,
-                                                          float* __restrict__ xs) {
-  const float* src = dx0 + (uint64_t)svals[blockIdx.x] * d;
-  float* dst = xs + (uint64_t)blockIdx.x * d;
-  if (vec) {
-    for (uint32_t c = threadIdx.x * kPerLane; c < d; c += kThreads * kPerLane)
-      st_g<f32x4>(dst + c, ld_nt<f32x4>(src + c));
-  } else {
-    for (uint32_t c = threadIdx.x; c < d; c += kThreads) st_g<float>(dst + c, ld_g<float>(src + c));
+// Up to kRankTokens tokens: the sorted position of every token position
+// directly, as the number of (key, position) pairs below its own.  Keys before
+// position p count when <= its key, keys after it when < it, so equal keys
+// keep increasing positions.  A block of kRankWaves waves ranks kRankPerBlock
+// positions against all n keys, staged through LDS kRankTile at a time: each
+// lane holds four keys, a compare gives 64 results as a scalar mask and the
+// counting is the scalar unit's (s_bcnt1), one vector instruction per 64
+// pairs.
+__global__ __launch_bounds__(kRankWaves * kWave) void rank_sort_kernel(
+    const uint32_t* __restrict__ tokens, uint32_t n, uint32_t vocab,
+    uint32_t* __restrict__ skeys, uint32_t* __restrict__ svals) {
+  __shared__ u32x4 s_keys[kRankTile / 4u];
+  const uint32_t lane = __lane_id();
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t p0 = blockIdx.x * kRankPerBlock + wave * kRankPerWave;
+  uint32_t key[kRankPerWave], rank[kRankPerWave];
+#pragma unroll
+  for (int i = 0; i < kRankPerWave; ++i) {
+    const uint32_t p = p0 + i < n ? p0 + i : n - 1u;
+    key[i] = __builtin_amdgcn_readfirstlane(clamp_token(ld_g<uint32_t>(tokens + p), vocab));
+    rank[i] = 0u;
+  }
+  for (uint32_t base = 0; base < n; base += kRankTile) {
+    if (base) __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < kRankTile / (4u * kRankWaves * kWave); ++j) {
+      const uint32_t v = j * (kRankWaves * kWave) + threadIdx.x;
+      const uint32_t q = base + 4u * v;
+      u32x4 k = {kPadKey, kPadKey, kPadKey, kPadKey};  // above every key
+      if (q + 4u <= n) {
+        k = (u32x4)ld_g<u32x4_a4>(tokens + q);
+        k.x = clamp_token(k.x, vocab);
+        k.y = clamp_token(k.y, vocab);
+        k.z = clamp_token(k.z, vocab);
+        k.w = clamp_token(k.w, vocab);
+      } else {
+        if (q < n) k.x = clamp_token(ld_g<uint32_t>(tokens + q), vocab);
+        if (q + 1u < n) k.y = clamp_token(ld_g<uint32_t>(tokens + q + 1u), vocab);
+        if (q + 2u < n) k.z = clamp_token(ld_g<uint32_t>(tokens + q + 2u), vocab);
+      }
+      s_keys[v] = k;
+    }
+    __syncthreads();
+    const uint32_t left = n - base;
+    const uint32_t quads = left < kRankTile ? (left + 1023u) / 1024u : kRankTile / 1024u;
+    for (uint32_t c4 = 0; c4 < quads; ++c4) {  // four groups of 256 keys, their reads together
+      u32x4 k[4];
+#pragma unroll
+      for (uint32_t c = 0; c < 4u; ++c) k[c] = s_keys[(c4 * 4u + c) * kWave + lane];
+#pragma unroll
+      for (uint32_t c = 0; c < 4u; ++c) {
+        const uint32_t q1 = base + (c4 * 4u + c + 1u) * 256u;  // the first position after the group
+#pragma unroll
+        for (int i = 0; i < kRankPerWave; ++i) {
+          const uint32_t bound = key[i] + (q1 <= p0 + i ? 1u : 0u);
+          rank[i] +=
+              (uint32_t)(__popcll(__ballot(k[c].x < bound)) + __popcll(__ballot(k[c].y < bound)) +
+                         __popcll(__ballot(k[c].z < bound)) + __popcll(__ballot(k[c].w < bound)));
+        }
+      }
+    }
+    // the group that holds p itself was taken as after it: its equals before p
+#pragma unroll
+    for (int i = 0; i < kRankPerWave; ++i) {
+      const uint32_t off = p0 + i - base;
+      if (off < kRankTile) {
+        const u32x4 k = s_keys[off / 256u * kWave + lane];
+        const uint32_t o = off % 256u, o0 = 4u * lane;
+        rank[i] += (uint32_t)(__popcll(__ballot(k.x == key[i] && o0 < o)) +
+                              __popcll(__ballot(k.y == key[i] && o0 + 1u < o)) +
+                              __popcll(__ballot(k.z == key[i] && o0 + 2u < o)) +
+                              __popcll(__ballot(k.w == key[i] && o0 + 3u < o)));
+      }
+    }
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int i = 0; i < kRankPerWave; ++i) {
+      if (p0 + i < n) {
+        skeys[rank[i]] = key[i];
+        svals[rank[i]] = p0 + i;
+      }
+    }
   }
 }
 
-// Block (p, tile): if sorted position p starts a run of equal keys, add the
-// run's rows (xs rows p.., in sorted order, which is increasing i) into
-// columns [tile*256, tile*256 + 256) of the key's embedding row.  vec:
-// d % 4 == 0 and g 16-byte aligned.
-__global__ __launch_bounds__(kTileCols) void run_kernel(float* __restrict__ g, uint32_t d,
-                                                        const float* __restrict__ xs,
-                                                        const uint32_t* __restrict__ skeys,
-                                                        uint32_t n, uint32_t vec) {
-  const uint32_t p = blockIdx.x;
-  const uint32_t t = skeys[p];
-  if (p > 0 && skeys[p - 1] == t) return;
-  // run end: the first sorted position with a larger key (binary search)
-  uint32_t lo = p, hi = n;  // skeys[lo] == t; hi is past the run
-  while (hi - lo > 1) {
-    const uint32_t mid = lo + ((hi - lo) >> 1);
-    if (skeys[mid] == t)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  const uint32_t len = hi - p;
-  const float* x = xs + (uint64_t)p * d;  // the run's rows, contiguous
-  if (len >= (uint32_t)kLongRun) {
-    const uint32_t c = blockIdx.y * kTileCols + threadIdx.x;
-    if (c >= d) return;
-    float* gp = g + (uint64_t)t * d + c;
-    float acc = ld_g<float>(gp);
-    uint32_t k = 0;
-    for (; k + kColRows <= len; k += kColRows) {
-      float v[kColRows];
-#pragma unroll
-      for (int j = 0; j < kColRows; ++j) v[j] = ld_g<float>(x + (uint64_t)(k + j) * d + c);
-#pragma unroll
-      for (int j = 0; j < kColRows; ++j) acc = acc + v[j];
-    }
-    if (k < len) {  // the last len % kColRows rows, loaded together as well
-      float v[kColRows];
-#pragma unroll
-      for (int j = 0; j < kColRows; ++j)
-        if (k + j < len) v[j] = ld_g<float>(x + (uint64_t)(k + j) * d + c);
-#pragma unroll
-      for (int j = 0; j < kColRows; ++j)
-        if (k + j < len) acc = acc + v[j];
-    }
-    st_g<float>(gp, acc);
-    return;
-  }
-  if (threadIdx.x >= kWave) return;  // a short run: the first wave, four columns per lane
-  const uint32_t c0 = blockIdx.y * kTileCols + threadIdx.x * kPerLane;
-  if (c0 >= d) return;
-  float* gp = g + (uint64_t)t * d + c0;
-  if (vec) {  // c0 + 4 <= d since d % 4 == 0
+// ---- the ordered adds -------------------------------------------------------
+// A run is a maximal stretch [start, end) of equal keys in the sorted order:
+// its positions svals[start..end) increase, and its rows dx0[svals[...]] are
+// added into the key's embedding row one after the other.
+
+// Row i of dx0, by a uniform i: the base stays in scalar registers and the
+// lane adds a 32-bit byte offset (a row is below 2^26 bytes).
+template <typename T>
+__device__ __forceinline__ T ld_row(const float* dx0, uint32_t d, uint32_t i, uint32_t byte_off) {
+  uint64_t base = (uint64_t)(dx0 + (uint64_t)i * d);
+  asm("" : "+s"(base));
+  return ld_nt<T>((const char*)base + byte_off);
+}
+
+// A run shorter than kLongRun that starts at sorted position p, columns
+// [256 * tile, +256) of the row, by one wave.  Rows are loaded kRowBatch at a
+// time before the first is added.  VEC (d % 4 == 0, embed_grad and dx0
+// 16-byte aligned): lane l owns columns 4l .. 4l + 3; otherwise columns
+// l, 64 + l, 128 + l, 192 + l, each access still one contiguous stretch.
+template <bool VEC>
+__device__ __forceinline__ void short_run(float* __restrict__ g, uint32_t d,
+                                          const float* __restrict__ dx0,
+                                          const uint32_t* __restrict__ skeys,
+                                          const uint32_t* __restrict__ svals, uint32_t n,
+                                          uint32_t p, uint32_t tile) {
+  const uint32_t lane = __lane_id();
+  const uint32_t q = p + lane < n ? p + lane : n - 1u;
+  const uint32_t k = ld_g<uint32_t>(skeys + q);
+  const uint32_t pos = ld_g<uint32_t>(svals + q);
+  const uint32_t t = __builtin_amdgcn_readfirstlane(k);
+  if (p != 0u && skeys[p - 1u] == t) return;  // not a run's start
+  const uint64_t other = ~__ballot(k == t && p + lane < n && lane < kLongRun);
+  const uint32_t len = (uint32_t)__ffsll((unsigned long long)other) - 1u;
+  if (len == kLongRun) return;  // long_run's
+  const uint32_t c0 = tile * kTileCols;
+  if constexpr (VEC) {
+    const uint32_t c = c0 + 4u * lane, cl = c < d ? c : d - 4u;  // past d: loaded, not stored
+    float* gp = g + (uint64_t)t * d + cl;
     f32x4 acc = ld_g<f32x4>(gp);
-    f32x4 v[kLongRun - 1];
+    for (uint32_t b = 0; b < len; b += kRowBatch) {
+      f32x4 v[kRowBatch];
 #pragma unroll
-    for (int j = 0; j < kLongRun - 1; ++j)
-      if ((uint32_t)j < len) v[j] = ld_g<f32x4>(x + (uint64_t)j * d + c0);
+      for (uint32_t j = 0; j < kRowBatch; ++j)
+        if (b + j < len)
+          v[j] = ld_row<f32x4>(dx0, d, __builtin_amdgcn_readlane(pos, b + j), cl * 4u);
 #pragma unroll
-    for (int j = 0; j < kLongRun - 1; ++j) {
-      if ((uint32_t)j < len) {
-        acc.x = acc.x + v[j].x;
-        acc.y = acc.y + v[j].y;
-        acc.z = acc.z + v[j].z;
-        acc.w = acc.w + v[j].w;
+      for (uint32_t j = 0; j < kRowBatch; ++j) {
+        if (b + j < len) {
+          acc.x = acc.x + v[j].x;
+          acc.y = acc.y + v[j].y;
+          acc.z = acc.z + v[j].z;
+          acc.w = acc.w + v[j].w;
+        }
       }
     }
-    st_g<f32x4>(gp, acc);
+    if (c < d) st_g<f32x4>(gp, acc);
   } else {
-    const int nc = d - c0 < (uint32_t)kPerLane ? (int)(d - c0) : kPerLane;
-    for (int c = 0; c < nc; ++c) {
-      float acc = ld_g<float>(gp + c);
-      for (uint32_t j = 0; j < len; ++j) acc = acc + ld_g<float>(x + (uint64_t)j * d + c0 + c);
-      st_g<float>(gp + c, acc);
+    // columns past d are clamped to the last one: loaded, never stored
+    uint32_t c[4];
+    float acc[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      c[u] = c0 + (uint32_t)u * kWave + lane;
+      acc[u] = ld_g<float>(g + (uint64_t)t * d + (c[u] < d ? c[u] : d - 1u));
+    }
+    for (uint32_t b = 0; b < len; b += kRowBatch) {
+      float v[kRowBatch][4];
+#pragma unroll
+      for (uint32_t j = 0; j < kRowBatch; ++j) {
+        if (b + j < len) {
+          const uint32_t i = __builtin_amdgcn_readlane(pos, b + j);
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            v[j][u] = ld_row<float>(dx0, d, i, (c[u] < d ? c[u] : d - 1u) * 4u);
+        }
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < kRowBatch; ++j) {
+        if (b + j < len) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) acc[u] = acc[u] + v[j][u];
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (c[u] < d) st_g<float>(g + (uint64_t)t * d + c[u], acc[u]);
+  }
+}
+
+// The run that holds sorted position p (a multiple of kLongRun), columns
+// [64 * ctile, +64), by the whole block: lane l of every wave owns column l.
+// Chunk c of the run is its rows [c * kColRows, +kColRows); wave w loads the
+// chunks w, w + kRunWaves, ... into registers ahead of their turn, and the running
+// sum goes from chunk to chunk through LDS, so up to kRunWaves * kColRows rows are in
+// flight while the additions keep the run's order.  A run of kLongRun rows
+// covers a multiple of kLongRun; the block at the first one takes the run.
+__device__ __forceinline__ void long_run(float* __restrict__ g, uint32_t d,
+                                         const float* __restrict__ dx0,
+                                         const uint32_t* __restrict__ skeys,
+                                         const uint32_t* __restrict__ svals, uint32_t n,
+                                         uint32_t p, uint32_t ctile, float* s_acc,
+                                         uint32_t* s_turn) {
+  const uint32_t lane = __lane_id();
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  // the kWave keys from p on, and those before it
+  const uint32_t kf = ld_g<uint32_t>(skeys + (p + lane < n ? p + lane : n - 1u));
+  const uint32_t kb = ld_g<uint32_t>(skeys + (p > lane ? p - 1u - lane : 0u));
+  const uint32_t t = __builtin_amdgcn_readfirstlane(kf);
+  const uint64_t fwd = ~__ballot(kf == t && p + lane < n);
+  const uint64_t bwd = ~__ballot(kb == t && lane < p && lane < kLongRun);
+  const uint32_t back = (uint32_t)__ffsll((unsigned long long)bwd) - 1u;
+  const uint32_t ahead = fwd ? (uint32_t)__ffsll((unsigned long long)fwd) - 1u : kWave;
+  if (back == kLongRun || back + ahead < kLongRun) return;  // an earlier block's, or short
+  const uint32_t start = p - back;
+  uint32_t end = p + ahead;
+  if (!fwd) {
+    // skeys[lo] == t and skeys[hi] != t (or hi == n), narrowed kWave probes at a time
+    uint32_t lo = p + kWave - 1u, hi = n;
+    while (hi - lo > 1u) {
+      const uint32_t step = (hi - lo + kWave - 1u) / kWave;
+      const uint64_t at = (uint64_t)lo + (uint64_t)(lane + 1u) * step;
+      const uint64_t miss = ~__ballot(at < hi && ld_g<uint32_t>(skeys + (at < hi ? at : lo)) == t);
+      const uint32_t m = (uint32_t)__ffsll((unsigned long long)miss) - 1u;  // the last probe is at hi or past it
+      const uint64_t top = (uint64_t)lo + (uint64_t)(m + 1u) * step;
+      if (top < hi) hi = (uint32_t)top;
+      lo += m * step;
+    }
+    end = hi;
+  }
+  if (threadIdx.x == 0) *s_turn = 0u;
+  __syncthreads();
+  const uint32_t c = ctile * kWave + lane;
+  const uint32_t cl = c < d ? c : d - 1u;  // lanes past d load the last column
+  const uint32_t chunks = (end - start + kColRows - 1u) / kColRows;
+  auto positions = [&](uint32_t ch) {  // chunk ch's, one per lane; past the run, its last
+    const uint32_t k = start + ch * kColRows + lane;
+    return ld_g<uint32_t>(svals + (k < end ? k : end - 1u));
+  };
+  uint32_t next = positions(wave);
+  for (uint32_t ch = wave; ch < chunks; ch += kRunWaves) {
+    const uint32_t k0 = start + ch * kColRows;
+    const uint32_t cnt = end - k0 < kColRows ? end - k0 : kColRows;
+    const uint32_t pos = next;
+    float v[kColRows];
+    if (cnt == kColRows) {
+#pragma unroll
+      for (uint32_t j = 0; j < kColRows; ++j)
+        v[j] = ld_row<float>(dx0, d, __builtin_amdgcn_readlane(pos, j), cl * 4u);
+    } else {
+#pragma unroll
+      for (uint32_t j = 0; j < kColRows; ++j)
+        if (j < cnt)
+          v[j] = ld_row<float>(dx0, d, __builtin_amdgcn_readlane(pos, j), cl * 4u);
+    }
+    next = positions(ch + kRunWaves);  // in flight while the wave waits its turn
+    float acc;
+    if (ch == 0u) {
+      acc = ld_g<float>(g + (uint64_t)t * d + cl);
+    } else {
+      while (__hip_atomic_load(s_turn, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) != ch)
+        __builtin_amdgcn_s_sleep(1);
+      acc = s_acc[lane];
+    }
+    if (cnt == kColRows) {
+#pragma unroll
+      for (uint32_t j = 0; j < kColRows; ++j) acc = acc + v[j];
+    } else {
+#pragma unroll
+      for (uint32_t j = 0; j < kColRows; ++j)
+        if (j < cnt) acc = acc + v[j];
+    }
+    if (ch + 1u == chunks) {
+      if (c < d) st_g<float>(g + (uint64_t)t * d + c, acc);
+    } else {
+      s_acc[lane] = acc;
+      if (lane == 0)
+        __hip_atomic_store(s_turn, ch + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
   }
+}
+
+// Sorted positions [p0, p1) (p0 a multiple of kLongRun): blocks below nlong
+// take the long runs, one (multiple of kLongRun, 64-column tile) each, and
+// come first because the longest run ends last; the others the short ones,
+// one wave per (position, 256-column tile), waves whose position starts no
+// short run leaving at once.
+template <bool VEC>
+__global__ __launch_bounds__(kRunWaves * kWave) void run_kernel(
+    float* __restrict__ g, uint32_t d, const float* __restrict__ dx0,
+    const uint32_t* __restrict__ skeys, const uint32_t* __restrict__ svals,
+    uint32_t n, uint32_t p0, uint32_t p1, uint32_t nlong) {
+  __shared__ float s_acc[kWave];
+  __shared__ uint32_t s_turn;
+  if (blockIdx.x < nlong) {
+    const uint32_t ctiles = (d + kWave - 1u) / kWave;
+    long_run(g, d, dx0, skeys, svals, n, p0 + blockIdx.x / ctiles * kLongRun,
+             blockIdx.x % ctiles, s_acc, &s_turn);
+    return;
+  }
+  const uint32_t tiles = (d + kTileCols - 1u) / kTileCols;
+  const uint32_t w = __builtin_amdgcn_readfirstlane((blockIdx.x - nlong) * kRunWaves +
+                                                    threadIdx.x / kWave);
+  const uint32_t p = p0 + w / tiles;
+  if (p < p1) short_run<VEC>(g, d, dx0, skeys, svals, n, p, w % tiles);
 }
 
 constexpr uint64_t kMaxFlatBlocks = 1u << 20;
 constexpr uint64_t kMaxPlanSegs = ((1ull << 32) - 1) / (kBlocksPerSeg * kWave);  // 4,194,303
-// gather_kernel and run_kernel launch one 256-lane block per token along x,
-// and a launch's work-items along one dimension must stay below 2^32.
-constexpr uint32_t kMaxTokens = (uint32_t)((1ull << 32) / kThreads) - 1u;  // 16,777,215
-static_assert(kTileCols == kThreads, "both per-token launches use 256-lane blocks");
+static_assert(kLongRun <= (uint32_t)kWave, "a lane for each row of a short run");
+constexpr uint32_t kMaxTokens = (1u << 24) - 1u;  // the call's limit (include/ark_grad.h)
+constexpr uint64_t kMaxRunBlocks = ((1ull << 32) - 1) / (kRunWaves * kWave);
 
 using ark::overlaps;
 
 using ark::StreamBuf;
 
-// Byte offsets of the scatter's workspace arrays, each 256-byte aligned:
-// the sorted keys and positions, for more than one tile a second pair that
-// the sort passes alternate with and the (digit, tile) counts, then the
-// copy of dx0 in sorted order.
+// Byte offsets of the scatter's workspace arrays, each 256-byte aligned: the
+// sorted keys and positions, and past kRankTokens a second pair that the radix
+// passes alternate with and the (digit, tile) counts.
 struct ScatterLayout {
-  uint32_t tiles = 0;  // kSortTile-item tiles; 1 = the one-block sort
-  size_t skeys = 0, svals = 0, keys = 0, vals = 0, counts = 0, xs = 0, bytes = 0;
+  uint32_t tiles = 0;  // kSortTile-item tiles
+  size_t skeys = 0, svals = 0, keys = 0, vals = 0, counts = 0, bytes = 0;
 };
 
-ScatterLayout scatter_layout(uint32_t n, uint32_t d) {
+ScatterLayout scatter_layout(uint32_t n) {
   ScatterLayout L;
   L.tiles = (n + kSortTile - 1) / kSortTile;
   const size_t arr = ark::align_up((size_t)n * 4, 256);
   size_t off = 0;
   L.skeys = off, off += arr;
   L.svals = off, off += arr;
-  if (L.tiles > 1) {
+  if (n > kRankTokens) {
     L.keys = off, off += arr;
     L.vals = off, off += arr;
     L.counts = off, off += ark::align_up((size_t)kRadix * L.tiles * 4, 256);
   }
-  L.xs = off, off += ark::align_up((size_t)n * d * 4, 256);
   L.bytes = off;
   return L;
+}
+
+// What the no-allocation call counts a batch as against its static array (the
+// size stated in include/ark_grad.h, which also allows for a copy of dx0):
+// never less than scatter_layout takes.
+size_t noalloc_need(uint32_t n, uint32_t d) {
+  const size_t arr = ark::align_up((size_t)n * 4, 256);
+  size_t need = 2 * arr + ark::align_up((size_t)n * d * 4, 256);
+  if (n > kSortTile)
+    need += 2 * arr + ark::align_up((size_t)kRadix * ((n + kSortTile - 1) / kSortTile) * 4, 256);
+  return need;
 }
 
 // Argument checks shared by the scatter's entry points; *skip is set when
@@ -669,10 +843,9 @@ int scatter_launch(float* embed_grad, uint32_t vocab, uint32_t d, const uint32_t
   while (end_bit < 32 && ((vocab - 1u) >> end_bit) != 0u) ++end_bit;
   uint32_t* skeys = (uint32_t*)(ws + L.skeys);
   uint32_t* svals = (uint32_t*)(ws + L.svals);
-  float* xs = (float*)(ws + L.xs);
-  if (L.tiles == 1) {
-    hipLaunchKernelGGL(block_sort_kernel, dim3(1), dim3(kSortThreads), 0, s, tokens, n, vocab,
-                       end_bit, skeys, svals);
+  if (n <= kRankTokens) {
+    hipLaunchKernelGGL(rank_sort_kernel, dim3((n + kRankPerBlock - 1) / kRankPerBlock),
+                       dim3(kRankWaves * kWave), 0, s, tokens, n, vocab, skeys, svals);
     ARK_HIP(hipGetLastError());
   } else {
     uint32_t* keys = (uint32_t*)(ws + L.keys);
@@ -702,13 +875,25 @@ int scatter_launch(float* embed_grad, uint32_t vocab, uint32_t d, const uint32_t
       in_v = out_v;
     }
   }
-  const uint32_t gvec = ((d % 4u) == 0 && (((uintptr_t)dx0 & 15u) == 0)) ? 1u : 0u;
-  hipLaunchKernelGGL(gather_kernel, dim3(n), dim3(kThreads), 0, s, dx0, svals, d, gvec, xs);
-  ARK_HIP(hipGetLastError());
-  const uint32_t vec = ((d % 4u) == 0 && (((uintptr_t)embed_grad & 15u) == 0)) ? 1u : 0u;
-  const dim3 grid(n, (d + kTileCols - 1) / kTileCols);
-  hipLaunchKernelGGL(run_kernel, grid, dim3(kTileCols), 0, s, embed_grad, d, xs, skeys, n, vec);
-  ARK_HIP(hipGetLastError());
+  const bool vec =
+      (d % 4u) == 0 && ((((uintptr_t)embed_grad | (uintptr_t)dx0) & 15u) == 0);
+  const uint64_t ctiles = (d + kWave - 1) / kWave, tiles = (d + kTileCols - 1) / kTileCols;
+  // a launch's work-items stay below 2^32: past that many positions, several
+  uint64_t per = kMaxRunBlocks / (ctiles + kLongRun * tiles / kRunWaves + 1u) * kLongRun;
+  if (per > n) per = n;
+  for (uint64_t p0 = 0; p0 < n; p0 += per) {
+    const uint64_t p1 = p0 + per < n ? p0 + per : n;
+    const uint64_t nlong = (p1 - p0 + kLongRun - 1) / kLongRun * ctiles;
+    const uint64_t nshort = ((p1 - p0) * tiles + kRunWaves - 1) / kRunWaves;
+    const dim3 grid((uint32_t)(nlong + nshort)), block(kRunWaves * kWave);
+    if (vec)
+      hipLaunchKernelGGL(run_kernel<true>, grid, block, 0, s, embed_grad, d, dx0, skeys, svals, n,
+                         (uint32_t)p0, (uint32_t)p1, (uint32_t)nlong);
+    else
+      hipLaunchKernelGGL(run_kernel<false>, grid, block, 0, s, embed_grad, d, dx0, skeys, svals,
+                         n, (uint32_t)p0, (uint32_t)p1, (uint32_t)nlong);
+    ARK_HIP(hipGetLastError());
+  }
   return ARK_OPT_OK;
 }
 
@@ -958,7 +1143,7 @@ int ark_grad_embed_scatter(float* embed_grad, uint32_t vocab, uint32_t d, const 
   if (rc || skip) return rc;
   invalidate_embed_units(embed_grad, vocab, d);
   hipStream_t s = (hipStream_t)stream;
-  const ScatterLayout L = scatter_layout(batch_seq, d);
+  const ScatterLayout L = scatter_layout(batch_seq);
   StreamBuf ws;
   hipError_t e = ws.alloc(L.bytes, s);
   if (e != hipSuccess) {
@@ -985,7 +1170,7 @@ int ark_grad_embed_scatter_final(float* embed_grad, uint32_t vocab, uint32_t d,
   if (skip) return ARK_OPT_OK;  // nothing changes; the units stay valid
   ark::DeviceGuard g(U.device);
   if (!g.ok) return fail(ARK_OPT_EHIP, "cannot select device %d", U.device);
-  const ScatterLayout L = scatter_layout(batch_seq, d);
+  const ScatterLayout L = scatter_layout(batch_seq);
   StreamBuf ws;
   hipError_t e = ws.alloc(L.bytes, U.stream);
   if (e != hipSuccess) {
@@ -1012,12 +1197,13 @@ int ark_grad_embed_scatter_noalloc(float* embed_grad, uint32_t vocab, uint32_t d
   bool skip = false;
   int rc = scatter_check(embed_grad, vocab, d, tokens, dx0, batch_seq, &skip);
   if (rc || skip) return rc;
-  const ScatterLayout L = scatter_layout(batch_seq, d);
-  if (L.bytes > (size_t)ARK_GRAD_SCRATCH_BYTES)
+  const ScatterLayout L = scatter_layout(batch_seq);
+  const size_t need = noalloc_need(batch_seq, d);
+  if (need > (size_t)ARK_GRAD_SCRATCH_BYTES)
     return fail(ARK_OPT_EINVAL,
-                "scatter of %u tokens x %u columns needs %zu bytes of workspace; the static "
+                "scatter of %u tokens x %u columns counts as %zu bytes of workspace; the static "
                 "scratch holds %llu (ark_grad_embed_scatter allocates instead)",
-                batch_seq, d, L.bytes, (unsigned long long)ARK_GRAD_SCRATCH_BYTES);
+                batch_seq, d, need, (unsigned long long)ARK_GRAD_SCRATCH_BYTES);
   hipStream_t s = (hipStream_t)stream;
   int dev = -1;
   hipError_t e = s ? hipStreamGetDevice(s, &dev) : hipGetDevice(&dev);

@@ -51,12 +51,12 @@ int ark_grad_plan_destroy(ark_grad_plan *plan);
  * t = tokens[i] < vocab ? tokens[i] : 0,
  *     embed_grad[t*d + j] += dx0[i*d + j]   for j < d.
  * Every element receives its additions in increasing i, as in the loop: the
- * positions are stably sorted by token on the device, the dx0 rows copied in
- * that order, and each token's rows added in order, column by column.
+ * positions are stably sorted by token on the device, and each token's rows
+ * added in that order, column by column.
  * embed_grad holds vocab*d floats, dx0 batch_seq*d, tokens batch_seq;
- * batch_seq < 2^24 (one 256-lane block per token), d <= 65535 * 256.
- * Stream ordered; the scratch it needs (a copy of dx0, 16 B per token and
- * the sort's) comes from the stream-ordered pool. */
+ * batch_seq < 2^24, d <= 65535 * 256.  Stream ordered; the scratch it needs
+ * (8 B per token, past 12288 tokens 16 B and 1 KiB per 4096) comes from the
+ * stream-ordered pool. */
 int ark_grad_embed_scatter(float *embed_grad, uint32_t vocab, uint32_t d,
                            const uint32_t *tokens, const float *dx0, uint32_t batch_seq,
                            void *stream);
@@ -113,12 +113,12 @@ int ark_grad_embed_scatter_final(float *embed_grad, uint32_t vocab, uint32_t d,
  * capture, tight serving loops, harnesses that forbid hipMalloc).  No
  * counterpart in the reference.  Its workspace is the static device array of
  * ARK_GRAD_SCRATCH_BYTES per GPU instead of the stream-ordered pool, so it
- * calls no hipMalloc, hipFree or other allocating routine.  The workspace is
+ * calls no hipMalloc, hipFree or other allocating routine.  A batch counts as
  *   8 * batch_seq bytes, plus 8 * batch_seq + 1024 * ceil(batch_seq / 4096)
  *   more when batch_seq > 4096, plus 4 * batch_seq * d,
  * each part rounded up to 256 bytes (a 2 x 2048-token batch at d = 768
- * needs 12.6 MB, at d = 2048 33.6 MB); a larger one is rejected with
- * ARK_OPT_EINVAL before anything is queued.
+ * counts as 12.6 MB, at d = 2048 as 33.6 MB; the call itself uses less); a
+ * larger one is rejected with ARK_OPT_EINVAL before anything is queued.
  *
  * Set-up: once per GPU the library looks the array's address up and creates
  * one event; ark_opt_create and ark_grad_plan_create do this for their GPU,

@@ -38,12 +38,11 @@ def _zipf_tokens(rng, n, vocab, extra=0):
                                              (256, 16, 12289, 3), (1, 8, 5000, 4),
                                              (70000, 8, 20000, 100), (100000, 4, 70001, 0)])
 def test_scatter_matches_oracle(vocab, d, n, extra):
-    """Up to 4096 tokens the positions are sorted by one block in LDS, past
-    that by one hist/scan/scatter launch triple per 8-bit digit over
-    4096-token tiles: two tiles exactly (8192), a one-token last tile
-    (4097, 12289), one pass (vocab 256 and 1), two, and three (vocab 70000
-    and 100000 take 17 key bits); vocab 32768 puts the largest real key on
-    the block sort's padding key."""
+    """Up to 12288 tokens the positions are sorted by counting over 4096-key
+    LDS tiles, past that by one hist/scan/scatter launch triple per 8-bit
+    digit over 4096-token tiles: two tiles exactly (8192), a one-token last
+    tile (4097, 12289), one pass (vocab 256), two, and three (vocab 70000 and
+    100000 take 17 key bits)."""
     torch = _torch()
     rng = np.random.default_rng(vocab + d + n)
     tokens = _zipf_tokens(rng, n, vocab, extra)
@@ -157,6 +156,32 @@ def test_scatter_run_lengths_at_the_path_boundaries(d):
     gg = torch.from_numpy(g).cuda()
     grad.embed_scatter(gg, torch.from_numpy(tokens.view(np.int32)).cuda(),
                        torch.from_numpy(dx0).cuda())
+    np.testing.assert_array_equal(_bits(gg).reshape(vocab, d), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("d,x_off", [(256, 0), (260, 0), (65, 0), (256, 1)])
+def test_scatter_run_lengths_around_the_block_shapes(d, x_off):
+    """Runs on both sides of where one wave hands over to a block (31, 32, 33
+    rows), of a wave's chunk (47 to 49, 95 to 97) and of the block's eight
+    chunks (383 to 385, 769), single rows between them, in a batch past one
+    4096-key tile; dx0 only 4-byte aligned with x_off = 1."""
+    torch = _torch()
+    rng = np.random.default_rng(d + x_off)
+    lengths = [7, 8, 9, 31, 32, 33, 47, 48, 49, 63, 64, 65, 95, 96, 97, 383, 384, 385, 769]
+    lengths += [1] * (4100 - sum(lengths))
+    vocab = 3000
+    ids = rng.permutation(vocab)[:len(lengths)]
+    tokens = np.concatenate([np.full(k, t, np.uint32) for k, t in zip(lengths, ids)])
+    tokens = tokens[rng.permutation(len(tokens))]
+    n = len(tokens)
+    dx0 = (rng.standard_normal((n, d)) * 10.0 ** rng.integers(-4, 4, (n, 1))).astype(np.float32)
+    g = rng.standard_normal((vocab, d)).astype(np.float32)
+    want = g.copy()
+    oracle.embed_scatter(want, tokens, dx0)
+    gg = torch.from_numpy(g).cuda()
+    xx = torch.zeros(n * d + x_off, device="cuda")[x_off:].view(n, d)
+    xx.copy_(torch.from_numpy(dx0))
+    grad.embed_scatter(gg, torch.from_numpy(tokens.view(np.int32)).cuda(), xx)
     np.testing.assert_array_equal(_bits(gg).reshape(vocab, d), want.view(np.uint32))
 
 
