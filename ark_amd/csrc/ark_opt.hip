@@ -239,16 +239,16 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
   const uint64_t parts = (nseg + spb - 1) / spb;
   if (parts > ark::kMaxParts)
     return fail(ARK_OPT_EINVAL, "too many elements (%llu segments)", (unsigned long long)nseg);
-  // Resident blocks per CU of the norm and AdamW passes;
-  // ARK_OPT_SUMSQ_BLOCKS_PER_CU=2..8 and ARK_OPT_ADAMW_BLOCKS_PER_CU=4..32
-  // override them, 0 lifts a cap (tuning knobs: results do not depend on
-  // them).
+  // Resident blocks per CU of the norm pass and one-wave rows per CU of the
+  // AdamW pass; ARK_OPT_SUMSQ_BLOCKS_PER_CU=2..8 and
+  // ARK_OPT_ADAMW_BLOCKS_PER_CU=4..32 (waves) override them, 0 lifts a cap
+  // (tuning knobs: results do not depend on them).
   int sumsq_per_cu = hp->grad_dtype == ARK_OPT_GRAD_F16 ? ark::kSumsqBlocksPerCuF16 : 0;
   if (const char* env = getenv("ARK_OPT_SUMSQ_BLOCKS_PER_CU")) {
     const int v = atoi(env);
     if (v == 0 || (v >= 2 && v <= 8)) sumsq_per_cu = v;
   }
-  int adamw_per_cu = ark::kAdamwBlocksPerCu;
+  int adamw_per_cu = ark::kAdamwWavesPerCu;
   if (const char* env = getenv("ARK_OPT_ADAMW_BLOCKS_PER_CU")) {
     const int v = atoi(env);
     if (v == 0 || (v >= 4 && v <= 32)) adamw_per_cu = v;

@@ -577,7 +577,7 @@ template <typename GT>
 __device__ __forceinline__ void adam_row(uint16_t* w, const GT* g, float* m, float* v,
                                          uint32_t valid, bool vec, float inv_t,
                                          float coef, const ElemConsts& k) {
-  const uint32_t e = threadIdx.x * 4u;
+  const uint32_t e = (threadIdx.x & 63u) * 4u;
   if (vec && valid == (uint32_t)kRow) {
     const typename GradIO<GT>::Raw4 gr = GradIO<GT>::load4(g + e);
     const u32x2 wr = ld_nt<u32x2>(w + e);
@@ -614,11 +614,24 @@ __device__ __forceinline__ void adam_row(uint16_t* w, const GT* g, float* m, flo
   }
 }
 
+// Block b's wave w takes row group * kAdamGroup + w * kAdamStride + b %
+// kAdamStride of the blocks' group b / kAdamStride: neighbouring rows run at the
+// same time on neighbouring blocks, hence on different XCDs, as with one row
+// per block, while a block dispatches kAdamWaves waves at once.  HBM bound;
+// what a skipped step pays is the dispatch.  Measured on MI355X, EKO-237M
+// (step / skipped step, us): one-wave blocks 842 / 287; blocks of two waves on
+// adjacent rows 877 / 191, on rows 64 apart 845 / 191; four waves 32 rows apart
+// 838 / 175, 16 apart 847, 64 apart 843, 128 apart 854; eight waves 852 / 181;
+// two rows per wave 850 / 155-190, four 872 / 140-160.
 template <typename GT>
-__global__ __launch_bounds__(64) void adamw_kernel(
+__global__ __launch_bounds__(64 * kAdamWaves) void adamw_kernel(
     const SegDesc* __restrict__ segs, const StepScalars* __restrict__ scal,
-    float beta1, float beta2, float eps) {
-  SegDesc d = segs[blockIdx.x / kRowsPerSeg];
+    float beta1, float beta2, float eps, uint32_t row0, uint32_t nrows) {
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t row = row0 + blockIdx.x / kAdamStride * kAdamGroup + wave * kAdamStride +
+                       blockIdx.x % kAdamStride;
+  if (row >= nrows) return;
+  SegDesc d = segs[row / kRowsPerSeg];
   StepScalars sc = *scal;
   // Every field used below is in registers before the first branch, so the
   // wave waits for one round trip of scalar loads rather than a chain of
@@ -628,7 +641,7 @@ __global__ __launch_bounds__(64) void adamw_kernel(
                "+s"(d.flags), "+s"(sc.applied), "+s"(sc.inv), "+s"(sc.coef), "+s"(sc.lr),
                "+s"(sc.lr_eff), "+s"(sc.c1), "+s"(sc.c2));
   if (!sc.applied) return;  // skipped step: training.rs:293-305
-  const uint32_t r0 = (blockIdx.x % kRowsPerSeg) * kRow;
+  const uint32_t r0 = (row % kRowsPerSeg) * kRow;
   if (r0 >= d.n) return;  // row past the end of a short segment
   const uint32_t valid = d.n - r0 < (uint32_t)kRow ? d.n - r0 : (uint32_t)kRow;
   ElemConsts c;
@@ -968,10 +981,10 @@ uint32_t sumsq_lds_for(uint32_t grad_dtype, int spb, int blocks) {
   return resident_lds_bytes(k, kBlock, blocks);
 }
 
-uint32_t adamw_lds_for(uint32_t grad_dtype, int blocks) {
+uint32_t adamw_lds_for(uint32_t grad_dtype, int waves) {
   const void* k = grad_dtype == ARK_OPT_GRAD_F16 ? (const void*)adamw_kernel<uint16_t>
                                                  : (const void*)adamw_kernel<float>;
-  return resident_lds_bytes(k, 64, blocks);
+  return resident_lds_bytes(k, 64 * kAdamWaves, (waves + kAdamWaves - 1) / kAdamWaves);
 }
 
 uint32_t finalize_leaves(uint32_t nparts) {
@@ -1006,14 +1019,23 @@ hipError_t launch_adamw(uint32_t grad_dtype, const SegDesc* segs, uint32_t nseg,
                         const StepScalars* scal, float beta1, float beta2,
                         float eps, uint32_t lds_bytes, hipStream_t stream) {
   if ((uint64_t)nseg > kMaxSegments) return hipErrorInvalidValue;
-  const dim3 grid(nseg * kRowsPerSeg), block(64);
-  if (grad_dtype == ARK_OPT_GRAD_F16)
-    hipLaunchKernelGGL((adamw_kernel<uint16_t>), grid, block, lds_bytes, stream, segs, scal,
-                       beta1, beta2, eps);
-  else
-    hipLaunchKernelGGL((adamw_kernel<float>), grid, block, lds_bytes, stream, segs, scal,
-                       beta1, beta2, eps);
-  return hipGetLastError();
+  const uint32_t nrows = nseg * kRowsPerSeg;
+  const dim3 block(64 * kAdamWaves);
+  // a launch's work-items stay below 2^32: the largest tables take two
+  constexpr uint32_t kMaxRows = (1u << 26) - kAdamGroup;
+  for (uint32_t row0 = 0; row0 < nrows; row0 += kMaxRows) {
+    const uint32_t rows = nrows - row0 < kMaxRows ? nrows - row0 : kMaxRows;
+    const dim3 grid((rows + kAdamGroup - 1) / kAdamGroup * kAdamStride);
+    if (grad_dtype == ARK_OPT_GRAD_F16)
+      hipLaunchKernelGGL((adamw_kernel<uint16_t>), grid, block, lds_bytes, stream, segs, scal,
+                         beta1, beta2, eps, row0, nrows);
+    else
+      hipLaunchKernelGGL((adamw_kernel<float>), grid, block, lds_bytes, stream, segs, scal, beta1,
+                         beta2, eps, row0, nrows);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_adamw_single(uint16_t* w, const float* g, float* m, float* v,

@@ -23,9 +23,9 @@
 // lane groups of 8 in index order.
 // adamw_kernel: one wave per 256-element row, lane l owning elements
 // [4l, 4l + 4): every load and store instruction of every array covers one
-// contiguous span (512 B of fp16, 1 KiB of fp32).  One-wave blocks over a
-// grid of ~a million rows measured fastest on MI355X for this mix of four
-// read streams and three write streams.
+// contiguous span (512 B of fp16, 1 KiB of fp32).  Blocks of four waves on
+// rows kAdamStride apart measured fastest on MI355X for this mix of four read
+// streams and three write streams (adamw_kernel).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -42,6 +42,9 @@ constexpr int kHalfSeg = kBlock * kVec;     // 2048
 static_assert(kSeg == 2 * kHalfSeg, "segment = two halves of 256 x 8");
 constexpr int kRow = 256;                   // adamw elements per wave
 constexpr int kRowsPerSeg = kSeg / kRow;    // 16
+constexpr uint32_t kAdamWaves = 4;          // adamw waves per block, one row each
+constexpr uint32_t kAdamStride = 32;        // rows between a block's waves
+constexpr uint32_t kAdamGroup = kAdamWaves * kAdamStride;  // rows of kAdamStride blocks
 constexpr int kFinThreads = 1024;           // finalize block
 
 // Segment descriptor flags.
@@ -112,7 +115,7 @@ constexpr uint32_t kFoldGroup = 64u;
 // past the real ones); out: padded_parts / kFoldGroup group sums.
 hipError_t launch_fold(uint32_t padded_parts, const double* in, double* out,
                        hipStream_t stream);
-// adamw grid: one wave per row, 16 rows per segment; the grid must stay
+// adamw: one wave per row, 16 rows per segment; rows and work-items must stay
 // below 2^32 work-items.
 constexpr uint64_t kMaxSegments = (1ull << 32) / (64ull * kRowsPerSeg) - 1;
 static_assert((kMaxSegments + 7) / 8 <= kMaxParts, "8 segments per norm block cover every table");
@@ -144,15 +147,14 @@ constexpr int kSumsqBlocksPerCuF16 = 7;
 // The dynamic LDS that holds the norm kernel for (grad_dtype, spb) at
 // `blocks` per CU (resident_lds_bytes; 0 = no cap).
 uint32_t sumsq_lds_for(uint32_t grad_dtype, int spb, int blocks);
-// Resident one-wave AdamW blocks per CU.  32 (every wave slot) over-issue
-// the pass's seven streams: on MI355X the EKO-237M pass takes 783.5 us
-// unbounded, 776.6 at 26 per CU, 762.5 at 20, 760.4-760.6 at 17 and 16,
-// 768 at 15 and 14 and 782 at 13; the 1.3B set's 4465-4480 us unbounded,
-// 4351 at 20, 4310-4323 at 17 and 16, 4283-4285 at 15 and 14.
-constexpr int kAdamwBlocksPerCu = 16;
-// The dynamic LDS that holds the AdamW kernel for grad_dtype at `blocks` per
-// CU (resident_lds_bytes; 0 = no cap).
-uint32_t adamw_lds_for(uint32_t grad_dtype, int blocks);
+// Resident AdamW waves per CU.  32 (every wave slot) over-issue the pass's
+// seven streams: on MI355X the EKO-237M step takes 857 us unbounded, 844 at 24
+// per CU, 833-855 at 20 and 16 (the spread is where the buffers lie), 866 at 12;
+// the 1.3B set's 4732 at 20, 4522-4588 at 16.
+constexpr int kAdamwWavesPerCu = 16;
+// The dynamic LDS that holds the AdamW kernel for grad_dtype at `waves` per
+// CU, rounded up to whole blocks (resident_lds_bytes; 0 = no cap).
+uint32_t adamw_lds_for(uint32_t grad_dtype, int waves);
 
 // The norm pass leaves the last kNormCachedBytes it reads (its lowest
 // blocks, where the AdamW pass starts) in the Infinity Cache and streams the
