@@ -65,10 +65,7 @@ struct ark_opt_handle {
   // one device allocation carved into the pieces below
   void* dev_mem = nullptr;
   SegDesc* d_segs = nullptr;
-  double* d_part_sum = nullptr;  // one partial per norm block, zero-padded
-  double* d_fold = nullptr;      // fold output when there are many partials
-  uint32_t padded_parts = 0;     // power of two >= parts when folding
-  uint32_t fin_leaves = 1;       // leaves per finalize thread
+  double* d_part_sum = nullptr;  // one slot per norm block
   ark_opt_state* d_state = nullptr;
   StepScalars* d_scal = nullptr;
   ark_opt_step_info* d_info = nullptr;
@@ -306,26 +303,9 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
   size_t off = 0;
   const size_t o_seg = off;
   off = align_up(off + sizeof(SegDesc) * (size_t)(nseg ? nseg : 1), 256);
-  // Partials: up to kFinTarget go straight to the finalize (kFinThreads *
-  // leaves doubles, zero past the real ones); more are first folded in
-  // aligned groups of kFoldGroup from a power-of-two zero-padded buffer.
-  const bool fold = parts > ark::kFinTarget;
-  uint32_t padded = 0, leaves = 0;
-  size_t psum_bytes = 0, fold_bytes = 0;
-  if (fold) {
-    padded = ark::kFoldGroup;
-    while (padded < parts) padded <<= 1;
-    psum_bytes = sizeof(double) * (size_t)padded;
-    leaves = ark::finalize_leaves(padded / ark::kFoldGroup);
-    fold_bytes = sizeof(double) * (size_t)ark::kFinThreads * leaves;
-  } else {
-    leaves = ark::finalize_leaves((uint32_t)parts);
-    psum_bytes = sizeof(double) * (size_t)ark::kFinThreads * leaves;
-  }
+  const size_t psum_bytes = sizeof(double) * (size_t)(parts ? parts : 1);
   const size_t o_psum = off;
   off = align_up(off + psum_bytes, 256);
-  const size_t o_fold = off;
-  off = align_up(off + fold_bytes, 256);
   const size_t o_state = off;
   off = align_up(off + sizeof(ark_opt_state), 256);
   const size_t o_scal = off;
@@ -345,9 +325,6 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
   char* base = (char*)h->dev_mem;
   h->d_segs = (SegDesc*)(base + o_seg);
   h->d_part_sum = (double*)(base + o_psum);
-  h->d_fold = fold ? (double*)(base + o_fold) : nullptr;
-  h->padded_parts = padded;
-  h->fin_leaves = leaves;
   h->d_state = (ark_opt_state*)(base + o_state);
   h->d_scal = (StepScalars*)(base + o_scal);
   h->d_info = (ark_opt_step_info*)(base + o_info);
@@ -372,8 +349,7 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
   StepScalars sc{};
   e = hipSuccess;
   if (nseg) e = hipMemcpy(h->d_segs, segs.data(), sizeof(SegDesc) * nseg, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemset(h->d_part_sum, 0, psum_bytes);
-  if (e == hipSuccess && fold) e = hipMemset(h->d_fold, 0, fold_bytes);
+  if (e == hipSuccess) e = hipMemset(h->d_part_sum, 0xFF, psum_bytes);  // every slot unset
   if (e == hipSuccess) e = hipMemcpy(h->d_state, &st, sizeof(st), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(h->d_scal, &sc, sizeof(sc), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
@@ -403,8 +379,8 @@ static int finish_info(ark_opt_handle* h, ark_opt_step_info* info) {
 
 namespace {
 
-// ark_opt_step with lr given on the host (lr_dev NULL) or read by the
-// finalize kernel from the device scalar lr_dev.
+// ark_opt_step with lr given on the host (lr_dev NULL) or read by the norm
+// pass's finalizer from the device scalar lr_dev.
 int step_impl(ark_opt_handle* h, float lr, const float* lr_dev, ark_opt_step_info* info) {
   DeviceGuard g(h->device);
   if (!g.ok) return fail(ARK_OPT_EHIP, "cannot select device %d", h->device);
@@ -417,23 +393,26 @@ int step_impl(ark_opt_handle* h, float lr, const float* lr_dev, ark_opt_step_inf
     ev = &h->ev[4 * h->pending];
     ARK_HIP(hipEventRecord(ev[0], h->stream));
   }
-  if (h->nseg) {
-    if (take_fresh_units(h)) {
-      // the gradients' producers already formed the tree's first level
-      ARK_HIP(ark::launch_units_reduce(h->spb, h->norm_blocks, h->d_units, h->d_segs, h->nseg,
-                                       h->d_part_sum, h->stream));
-    } else {
-      ARK_HIP(ark::launch_sumsq(h->hp.grad_dtype, h->spb, h->norm_blocks, h->d_segs,
-                                h->nseg, h->d_state, h->d_part_sum, h->nt_from, h->sumsq_lds,
-                                h->stream));
-    }
-    if (h->d_fold)
-      ARK_HIP(ark::launch_fold(h->padded_parts, h->d_part_sum, h->d_fold, h->stream));
+  ark::FinalizeArgs fin{};
+  fin.part = h->d_part_sum;
+  fin.nparts = h->norm_blocks;
+  fin.lr = lr;
+  fin.lr_ptr = lr_dev;
+  fin.state = h->d_state;
+  fin.scal = h->d_scal;
+  fin.info = h->d_info;
+  fin.hp = h->hp;
+  if (take_fresh_units(h)) {
+    // the gradients' producers already formed the tree's first level
+    ARK_HIP(ark::launch_units_reduce(h->spb, h->d_units, h->d_segs, h->nseg, fin, h->stream));
+  } else {
+    ARK_HIP(ark::launch_sumsq(h->hp.grad_dtype, h->spb, h->d_segs, h->nseg, h->nt_from, fin,
+                              h->sumsq_lds, h->stream));
   }
-  if (ev) ARK_HIP(hipEventRecord(ev[1], h->stream));
-  ARK_HIP(ark::launch_finalize(h->fin_leaves, h->d_fold ? h->d_fold : h->d_part_sum, h->hp,
-                               lr, lr_dev, h->d_state, h->d_scal, h->d_info, h->stream));
-  if (ev) ARK_HIP(hipEventRecord(ev[2], h->stream));
+  if (ev) {
+    ARK_HIP(hipEventRecord(ev[1], h->stream));
+    ARK_HIP(hipEventRecord(ev[2], h->stream));
+  }
   if (h->nseg) {
     ARK_HIP(ark::launch_adamw(h->hp.grad_dtype, h->d_segs, h->nseg, h->d_scal,
                               h->hp.beta1, h->hp.beta2, h->hp.eps, h->adamw_lds, h->stream));

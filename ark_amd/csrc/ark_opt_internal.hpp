@@ -53,9 +53,9 @@ void opt_units_set_fresh(ark_opt_handle* h, bool fresh);
 // (opt_units_invalidate, the other writers' side, is in ark_common.hpp.)
 
 // units -> one partial per norm block of spb segments, exactly what
-// sumsq_kernel would write for the same gradients (launch_sumsq's part_sum).
-hipError_t launch_units_reduce(int spb, uint32_t nblocks, const double* units,
-                               const SegDesc* segs, uint32_t nseg, double* part_sum,
-                               hipStream_t stream);
+// sumsq_kernel would publish for the same gradients, and the finalizer as in
+// launch_sumsq.
+hipError_t launch_units_reduce(int spb, const double* units, const SegDesc* segs, uint32_t nseg,
+                               const FinalizeArgs& fin, hipStream_t stream);
 
 }  // namespace ark

@@ -191,6 +191,182 @@ __device__ __forceinline__ double butterfly_from(double x) {
 
 constexpr int log2i(int v) { return v <= 1 ? 0 : 1 + log2i(v / 2); }
 
+// ---- kernel 1's finalizer ----------------------------------------------------
+// Block 0 of the norm pass finishes the step's scalars in the same launch: it
+// takes every block's partial as it appears and runs the AMP and clip
+// decisions.  It is one block and the only one that waits, for blocks that wait
+// for nothing, so the grid always drains.  A partial travels in its own slot, a
+// 64-bit agent-scope store and load (both pass the XCDs' L2s by) of a slot that
+// holds kUnset until then, so no fence orders anything; the finalizer puts
+// kUnset back for the next step.  What it costs is the time from the last
+// partial to the scalars.  Measured on MI355X, norm pass to scalars, us (a norm
+// kernel, past 8192 partials a fold, and a one-block finalize before): one
+// 768 x 768 tensor 4.8 (3.2 + 3.3 and a launch between), one layer 7.8 (5.7 +
+// 4.0), EKO-237M 76.4 (73.3 + 4.7 + 4.6), from units 7.8 (4.8 + 4.8), the 1.3B
+// set 373 (373 + 5 + 5).
+
+constexpr uint64_t kUnset = ~0ull;  // a NaN that publish() never stores
+
+__device__ __forceinline__ void publish(double* slot, double x) {
+  uint64_t b = __builtin_bit_cast(uint64_t, x);
+  if (b == kUnset) b = 0x7FF8000000000000ull;
+  __hip_atomic_store((ARK_GLOBAL uint64_t*)slot, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Pairwise tree over the 64 * R partials of one group (0 past nparts) when all
+// have been published.  Lane l takes partials l, 64 + l, ...: every access is
+// one contiguous stretch, and transpose_reduce turns the R trees over the lanes
+// into one value per lane, whose index has its bits in the lane's reversed.
+template <int R>
+__device__ __forceinline__ double take_group(double* __restrict__ part, uint32_t nparts,
+                                             uint32_t group, uint32_t lane) {
+  ARK_GLOBAL uint64_t* p = (ARK_GLOBAL uint64_t*)part;
+  const uint32_t i0 = group * 64u * R + lane;
+  uint64_t v[R];
+  for (;;) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      v[r] = 0ull;
+      if (i0 + r * 64u < nparts)
+        v[r] = __hip_atomic_load(p + i0 + r * 64u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    bool ready = true;
+#pragma unroll
+    for (int r = 0; r < R; ++r) ready = ready && v[r] != kUnset;
+    if (__all(ready)) break;
+    __builtin_amdgcn_s_sleep(1);
+  }
+  double q[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (i0 + r * 64u < nparts)
+      __hip_atomic_store(p + i0 + r * 64u, kUnset, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    q[r] = __builtin_bit_cast(double, v[r]);
+  }
+  int idx = 0;
+  transpose_reduce<R, 0>(q, (int)lane, idx);
+  double x = butterfly_from<log2i(R)>(q[0]);
+#pragma unroll
+  for (int st = log2i(R) - 1; st >= 0; --st) x = x + __shfl_xor(x, 1 << st);
+  return x;
+}
+
+// The root of the tree over the nparts partials, in wave 0.  The norm blocks
+// run from the last to the first, and so do the groups here; sums holds
+// kFinGroups values in LDS.
+template <int R>
+__device__ __forceinline__ double take_all(double* __restrict__ part, uint32_t nparts,
+                                           double* sums) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t groups = (nparts + 64u * R - 1u) / (64u * R);
+  for (uint32_t i = threadIdx.x; i < kFinGroups; i += kBlock)
+    if (i >= groups) sums[i] = 0.0;
+  for (uint32_t k = wave; k < groups; k += kBlock / 64) {
+    const double x = take_group<R>(part, nparts, groups - 1u - k, lane);
+    if (lane == 0) sums[groups - 1u - k] = x;
+  }
+  __syncthreads();
+  if (wave != 0) return 0.0;
+  constexpr int kPer = (int)kFinGroups / 64;
+  double q[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) q[j] = sums[lane * kPer + j];
+#pragma unroll
+  for (int w = kPer / 2; w >= 1; w /= 2)
+#pragma unroll
+    for (int j = 0; j < w; ++j) q[j] = q[2 * j] + q[2 * j + 1];
+  return butterfly_from<0>(q[0]);
+}
+
+__device__ inline uint32_t amp_skip(const ark_opt_hparams& hp, ark_opt_state& st) {
+  // training.rs:294-301 (and :231-236 for the logits-gradient check)
+  st.loss_scale = fmaxf(st.loss_scale * 0.5f, hp.loss_scale_min);
+  st.clean_steps = 0u;
+  st.skipped_steps += 1u;
+  st.consecutive_nonfinite += 1u;
+  if (st.consecutive_nonfinite > hp.max_consecutive_nonfinite) {
+    st.early_stop = 1u;
+    return ARK_OPT_EARLY_STOP;
+  }
+  return ARK_OPT_OK;
+}
+
+// lr_ptr: when not NULL, this step's learning rate is *lr_ptr (read as the
+// kernel runs) instead of lr; a non-finite one makes the step a no-op that
+// reports ARK_OPT_EINVAL.  kMaxR: partials per lane in the largest groups (the
+// norm pass takes 8, whose registers its blocks have anyway).
+template <int kMaxR>
+__device__ __forceinline__ void finalize_step(const FinalizeArgs& a, double* sums) {
+  // what does not depend on the sum first, while the partials are on their way
+  const ark_opt_hparams hp = a.hp;
+  const float lr = a.lr_ptr ? *a.lr_ptr : a.lr;
+  ark_opt_state st = *a.state;
+  const float inv = 1.0f / st.loss_scale;  // training.rs:244
+  const float lr_eff = lr_eff_of(lr, hp.beta1, hp.beta2, st.t + 1u);
+  double sumsq;
+  // a round of the waves takes all partials of a small table, and few rounds
+  // those of a large one
+  if (a.nparts <= kBlock)
+    sumsq = take_all<1>(a.part, a.nparts, sums);
+  else if (a.nparts <= 4u * kBlock)
+    sumsq = take_all<4>(a.part, a.nparts, sums);
+  else
+    sumsq = take_all<kMaxR>(a.part, a.nparts, sums);
+  if (threadIdx.x != 0) return;
+
+  const bool any_bad = __builtin_isnan(sumsq);
+  StepScalars sc = {};
+  ark_opt_step_info out = {};
+  sc.c1 = 1.0f - hp.beta1;
+  sc.c2 = 1.0f - hp.beta2;
+  sc.lr = lr;
+  sc.coef = 1.0f;
+  out.lr = lr;
+  out.clip_coef = 1.0f;
+  out.status = ARK_OPT_OK;
+  out.inv_scale = inv;
+  if (st.early_stop) {
+    out.status = ARK_OPT_EARLY_STOP;
+  } else if (!(fabsf(lr) <= 3.402823466e38f)) {  // a non-finite lr: nothing changes
+    out.status = ARK_OPT_EINVAL;
+    sc.lr = 0.0f;
+  } else {
+    const float scale = st.loss_scale;
+    sc.inv = inv;
+    out.grad_sumsq = sumsq;
+    const float norm = sqrtf((float)sumsq);  // optimizer.rs:145
+    out.grad_norm = norm;
+    if (any_bad) {  // training.rs:293-305: no update, t unchanged
+      out.nonfinite = 1;
+      out.status = (int32_t)amp_skip(hp, st);
+    } else {
+      const bool clipped = (norm > hp.grad_clip) && (norm > 0.0f);  // :148
+      const float coef = clipped ? hp.grad_clip / norm : 1.0f;     // :149
+      st.t += 1u;                                                   // :172
+      sc.applied = 1u;
+      sc.clipped = clipped ? 1u : 0u;
+      sc.coef = coef;
+      sc.lr_eff = lr_eff;
+      out.applied = 1;
+      out.clipped = clipped ? 1 : 0;
+      out.clip_coef = coef;
+      out.lr_eff = lr_eff;
+      st.clean_steps += 1u;           // training.rs:317
+      st.consecutive_nonfinite = 0u;  // :318
+      if (st.clean_steps >= hp.scale_up_every) {                     // :319
+        const float nueva = fminf(scale * 2.0f, hp.loss_scale_max);  // :320
+        if (nueva > scale) st.loss_scale = nueva;                     // :321
+        st.clean_steps = 0u;                                          // :325
+      }
+    }
+  }
+  out.state = st;
+  *a.state = st;
+  *a.scal = sc;
+  *a.info = out;
+}
+
 // ---- kernel 1: sum of squares + non-finite flag -----------------------------
 
 // One batch of kRed full, 16-byte aligned segments (descriptors d) into
@@ -227,8 +403,8 @@ __device__ __forceinline__ void fast_batch(const SegDesc (&dsc)[kRed], int tid, 
   }
 }
 
-// Block b covers segments [b*SPB, b*SPB + SPB) (SPB <= 8) and writes the
-// pairwise tree of their 2*SPB half-segment sums: an aligned subtree of the
+// Block 0 is the finalizer.  The others cover segments [b*SPB, b*SPB + SPB)
+// (SPB <= 8) each, b counted from the last, and publish the pairwise tree of their 2*SPB half-segment sums: an aligned subtree of the
 // global tree.  A block that saw an inf or NaN gradient writes NaN, so the
 // global sum is NaN exactly when some gradient is non-finite (training.rs:291).
 // Blocks from nt_from up read with non-temporal loads: they run first, and
@@ -238,13 +414,18 @@ __device__ __forceinline__ void fast_batch(const SegDesc (&dsc)[kRed], int tid, 
 template <typename GT, int SPB>
 __global__ __launch_bounds__(kBlock) void sumsq_kernel(
     const SegDesc* __restrict__ segs, uint32_t nseg, const ark_opt_state* __restrict__ state,
-    double* __restrict__ part_sum, uint32_t nt_from) {
+    uint32_t nt_from, FinalizeArgs fin) {
   static_assert(SPB >= 1 && SPB <= 8 && (SPB & (SPB - 1)) == 0, "1, 2, 4 or 8 segments");
   constexpr int V = 2 * SPB;  // half-segment values per lane
   // segments whose loads are in flight together (register budget)
   constexpr int kLoadMax = sizeof(GT) == 2 ? 8 : 4;
   constexpr int kLoad = kLoadMax < SPB ? kLoadMax : SPB;
   __shared__ double lds[kBlock / 64][V];
+  __shared__ double sums[kFinGroups];
+  if (blockIdx.x == 0) {
+    finalize_step<8>(fin, sums);
+    return;
+  }
 
   // Blocks run in reverse: the last block, which usually holds the ragged
   // tail of the table, starts first instead of trailing the grid.
@@ -335,7 +516,7 @@ __global__ __launch_bounds__(kBlock) void sumsq_kernel(
     for (int st = 0; st < log2i(V); ++st) x = x + __shfl_xor(x, 1 << st);
     // sq16 blocks: a non-finite sum is exactly a non-finite gradient
     const bool nonfinite = any_bad || (sq16 && !__builtin_isfinite(x));
-    if (tid == 0) part_sum[blk] = nonfinite ? __builtin_nan("") : x;
+    if (tid == 0) publish(fin.part + blk, nonfinite ? __builtin_nan("") : x);
   }
 }
 
@@ -347,20 +528,28 @@ __global__ __launch_bounds__(kBlock) void sumsq_kernel(
 // the perfect binary tree sumsq_kernel forms over the block's elements, so
 // the partial has the same bits; a NaN unit (a non-finite gradient) makes the
 // partial NaN.
+// Block 0 is the finalizer, the waves of the others take the partials.
 template <int SPB>
-__global__ __launch_bounds__(64) void units_reduce_kernel(const double* __restrict__ units,
-                                                          const SegDesc* __restrict__ segs,
-                                                          uint32_t nseg,
-                                                          double* __restrict__ part_sum) {
+__global__ __launch_bounds__(kBlock) void units_reduce_kernel(const double* __restrict__ units,
+                                                              const SegDesc* __restrict__ segs,
+                                                              uint32_t nseg, FinalizeArgs fin) {
+  __shared__ double sums[kFinGroups];
+  if (blockIdx.x == 0) {
+    finalize_step<16>(fin, sums);
+    return;
+  }
   constexpr int U = SPB * kUnitsPerSeg;     // 16 .. 128 units per block
   constexpr int K = U >= 64 ? U / 64 : 1;   // units per lane
   constexpr int L = U >= 64 ? 64 : U;       // lanes holding units
   static_assert(K <= kUnitsPerSeg, "a lane's units lie in one segment");
-  const uint32_t lane = threadIdx.x;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t blk = (gridDim.x - 1u - blockIdx.x) * (kBlock / 64) +
+                       __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (blk >= fin.nparts) return;
   double x = 0.0;
   if (lane < (uint32_t)L) {
     const uint32_t u0 = lane * K;
-    const uint32_t s = blockIdx.x * SPB + u0 / kUnitsPerSeg;
+    const uint32_t s = blk * SPB + u0 / kUnitsPerSeg;
     double q[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) q[k] = 0.0;
@@ -379,131 +568,10 @@ __global__ __launch_bounds__(64) void units_reduce_kernel(const double* __restri
   }
 #pragma unroll
   for (int st = 0; st < log2i(L); ++st) x = x + __shfl_xor(x, 1 << st);
-  if (lane == 0) part_sum[blockIdx.x] = x;
+  if (lane == 0) publish(fin.part + blk, x);
 }
 
-// ---- kernel 2: finalize ----------------------------------------------------
-
-// Pairwise tree over p[0, L) (p 16-byte aligned, L a power of two).
-template <int L>
-__device__ __forceinline__ double leaf_tree(const double* __restrict__ p) {
-  if constexpr (L == 1) {
-    return p[0];
-  } else if constexpr (L == 2) {
-    typedef double f64x2 __attribute__((ext_vector_type(2)));
-    const f64x2 v = *(const ARK_GLOBAL f64x2*)p;
-    return v.x + v.y;
-  } else {
-    const double a = leaf_tree<L / 2>(p);
-    const double b = leaf_tree<L / 2>(p + L / 2);
-    return a + b;
-  }
-}
-
-// Many partials: one wave per aligned group of kFoldGroup partials writes the
-// group's pairwise tree (again an aligned subtree), so the single-block
-// finalize never reads more than kFinTarget values.
-__global__ __launch_bounds__(kFoldGroup) void fold_kernel(const double* __restrict__ in,
-                                                          double* __restrict__ out) {
-  double x = in[blockIdx.x * kFoldGroup + threadIdx.x];
-  x = butterfly_from<0>(x);
-  if (threadIdx.x == 0) out[blockIdx.x] = x;
-}
-
-__device__ inline uint32_t amp_skip(const ark_opt_hparams& hp, ark_opt_state& st) {
-  // training.rs:294-301 (and :231-236 for the logits-gradient check)
-  st.loss_scale = fmaxf(st.loss_scale * 0.5f, hp.loss_scale_min);
-  st.clean_steps = 0u;
-  st.skipped_steps += 1u;
-  st.consecutive_nonfinite += 1u;
-  if (st.consecutive_nonfinite > hp.max_consecutive_nonfinite) {
-    st.early_stop = 1u;
-    return ARK_OPT_EARLY_STOP;
-  }
-  return ARK_OPT_OK;
-}
-
-// part_sum holds kFinThreads * L partials, zero past the last block's.
-// lr_ptr: when not NULL, this step's learning rate is *lr_ptr (read as the
-// kernel runs) instead of lr; a non-finite one makes the step a no-op that
-// reports ARK_OPT_EINVAL.
-template <int L>
-__global__ __launch_bounds__(kFinThreads) void finalize_kernel(
-    const double* __restrict__ part_sum, ark_opt_hparams hp, float lr,
-    const float* __restrict__ lr_ptr, ark_opt_state* __restrict__ state,
-    StepScalars* __restrict__ scal, ark_opt_step_info* __restrict__ info) {
-  __shared__ double wsum[kFinThreads / 64];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-
-  double x = leaf_tree<L>(part_sum + (uint32_t)tid * L);
-  x = butterfly_from<0>(x);
-  if (lane == 0) wsum[wave] = x;
-  __syncthreads();
-  if (wave != 0) return;
-  double y = lane < kFinThreads / 64 ? wsum[lane] : 0.0;
-#pragma unroll
-  for (int s = 0; s < log2i(kFinThreads / 64); ++s) y = y + __shfl_xor(y, 1 << s);
-  if (lane != 0) return;
-
-  if (lr_ptr) lr = *lr_ptr;
-  const double sumsq = y;
-  const bool any_bad = __builtin_isnan(sumsq);
-  ark_opt_state st = *state;
-  StepScalars sc = {};
-  ark_opt_step_info out = {};
-  sc.c1 = 1.0f - hp.beta1;
-  sc.c2 = 1.0f - hp.beta2;
-  sc.lr = lr;
-  sc.coef = 1.0f;
-  out.lr = lr;
-  out.clip_coef = 1.0f;
-  out.status = ARK_OPT_OK;
-  if (st.early_stop) {
-    out.status = ARK_OPT_EARLY_STOP;
-    out.inv_scale = 1.0f / st.loss_scale;
-  } else if (!(fabsf(lr) <= 3.402823466e38f)) {  // a non-finite lr: nothing changes
-    out.status = ARK_OPT_EINVAL;
-    out.inv_scale = 1.0f / st.loss_scale;
-    sc.lr = 0.0f;
-  } else {
-    const float scale = st.loss_scale;
-    const float inv = 1.0f / scale;  // training.rs:244
-    sc.inv = inv;
-    out.inv_scale = inv;
-    out.grad_sumsq = sumsq;
-    const float norm = sqrtf((float)sumsq);  // optimizer.rs:145
-    out.grad_norm = norm;
-    if (any_bad) {  // training.rs:293-305: no update, t unchanged
-      out.nonfinite = 1;
-      out.status = (int32_t)amp_skip(hp, st);
-    } else {
-      const bool clipped = (norm > hp.grad_clip) && (norm > 0.0f);  // :148
-      const float coef = clipped ? hp.grad_clip / norm : 1.0f;     // :149
-      st.t += 1u;                                                   // :172
-      sc.applied = 1u;
-      sc.clipped = clipped ? 1u : 0u;
-      sc.coef = coef;
-      sc.lr_eff = lr_eff_of(lr, hp.beta1, hp.beta2, st.t);
-      out.applied = 1;
-      out.clipped = clipped ? 1 : 0;
-      out.clip_coef = coef;
-      out.lr_eff = sc.lr_eff;
-      st.clean_steps += 1u;           // training.rs:317
-      st.consecutive_nonfinite = 0u;  // :318
-      if (st.clean_steps >= hp.scale_up_every) {                     // :319
-        const float nueva = fminf(scale * 2.0f, hp.loss_scale_max);  // :320
-        if (nueva > scale) st.loss_scale = nueva;                     // :321
-        st.clean_steps = 0u;                                          // :325
-      }
-    }
-  }
-  out.state = st;
-  *state = st;
-  *scal = sc;
-  *info = out;
-}
+// ---- the logits-gradient skip -----------------------------------------------
 
 __global__ void record_overflow_kernel(ark_opt_hparams hp,
                                        ark_opt_state* __restrict__ state,
@@ -904,10 +972,10 @@ int sumsq_spb(uint64_t nseg, uint32_t grad_dtype) {
   // EKO-237M: each block's descriptor load then stands alone in front of
   // its data loads), as are 16 and 32.
   // fp32 gradients: 8.  Such a handle's norm usually comes from the units
-  // the gradient hand-off wrote (units_reduce_kernel: one wave per block
-  // reads 16 doubles per segment), whose cost is per block, not per byte: at
-  // EKO-237M 4.5 us with 8 segments per block and no fold, against 8.5 us
-  // plus a 4.5 us fold with 2 (the reading pass gains 4.6 us with 2).
+  // the gradient hand-off wrote (units_reduce_kernel: one wave per partial
+  // reads 16 doubles per segment), whose cost is per partial, not per byte: at
+  // EKO-237M 4.5 us with 8 segments per partial against 8.5 us with 2, and
+  // four times the partials to finish (the reading pass gains 4.6 us with 2).
   // Larger blocks only when the partials would exceed kMaxParts (beyond
   // 2^31 elements); 8 covers every table kMaxSegments allows.  A small table
   // gets smaller blocks until the grid has two blocks per CU (512): the pass
@@ -919,22 +987,13 @@ int sumsq_spb(uint64_t nseg, uint32_t grad_dtype) {
   return spb;
 }
 
-hipError_t launch_fold(uint32_t padded_parts, const double* in, double* out,
-                       hipStream_t stream) {
-  if (padded_parts % kFoldGroup) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(fold_kernel, dim3(padded_parts / kFoldGroup), dim3(kFoldGroup), 0,
-                     stream, in, out);
-  return hipGetLastError();
-}
-
-hipError_t launch_sumsq(uint32_t grad_dtype, int spb, uint32_t nblocks,
-                        const SegDesc* segs, uint32_t nseg, const ark_opt_state* state,
-                        double* part_sum, uint32_t nt_from, uint32_t lds_bytes,
+hipError_t launch_sumsq(uint32_t grad_dtype, int spb, const SegDesc* segs, uint32_t nseg,
+                        uint32_t nt_from, const FinalizeArgs& fin, uint32_t lds_bytes,
                         hipStream_t stream) {
-  const dim3 grid(nblocks), block(kBlock);
+  const dim3 grid(fin.nparts + 1u), block(kBlock);
 #define ARK_SUMSQ(GT, SPB)                                                                \
   hipLaunchKernelGGL((sumsq_kernel<GT, SPB>), grid, block, lds_bytes, stream, segs, nseg, \
-                     state, part_sum, nt_from)
+                     fin.state, nt_from, fin)
   switch (spb * 2 + (grad_dtype == ARK_OPT_GRAD_F16 ? 0 : 1)) {
     case 2: ARK_SUMSQ(uint16_t, 1); break;
     case 4: ARK_SUMSQ(uint16_t, 2); break;
@@ -950,13 +1009,11 @@ hipError_t launch_sumsq(uint32_t grad_dtype, int spb, uint32_t nblocks,
   return hipGetLastError();
 }
 
-hipError_t launch_units_reduce(int spb, uint32_t nblocks, const double* units,
-                               const SegDesc* segs, uint32_t nseg, double* part_sum,
-                               hipStream_t stream) {
-  const dim3 grid(nblocks), block(64);
+hipError_t launch_units_reduce(int spb, const double* units, const SegDesc* segs, uint32_t nseg,
+                               const FinalizeArgs& fin, hipStream_t stream) {
+  const dim3 grid((fin.nparts + kBlock / 64 - 1u) / (kBlock / 64) + 1u), block(kBlock);
 #define ARK_UNITS(SPB)                                                                     \
-  hipLaunchKernelGGL((units_reduce_kernel<SPB>), grid, block, 0, stream, units, segs, nseg, \
-                     part_sum)
+  hipLaunchKernelGGL((units_reduce_kernel<SPB>), grid, block, 0, stream, units, segs, nseg, fin)
   switch (spb) {
     case 1: ARK_UNITS(1); break;
     case 2: ARK_UNITS(2); break;
@@ -991,28 +1048,6 @@ uint32_t finalize_leaves(uint32_t nparts) {
   uint32_t L = 1;
   while ((uint64_t)L * kFinThreads < nparts) L <<= 1;
   return L;
-}
-
-hipError_t launch_finalize(uint32_t leaves, const double* part_sum,
-                           const ark_opt_hparams& hp, float lr, const float* lr_ptr,
-                           ark_opt_state* state, StepScalars* scal,
-                           ark_opt_step_info* info, hipStream_t stream) {
-  const dim3 grid(1), block(kFinThreads);
-#define ARK_FIN(L)                                                                   \
-  hipLaunchKernelGGL((finalize_kernel<L>), grid, block, 0, stream, part_sum, hp, lr, \
-                     lr_ptr, state, scal, info)
-  switch (leaves) {
-    case 1: ARK_FIN(1); break;
-    case 2: ARK_FIN(2); break;
-    case 4: ARK_FIN(4); break;
-    case 8: ARK_FIN(8); break;
-    case 16: ARK_FIN(16); break;
-    case 32: ARK_FIN(32); break;
-    case 64: ARK_FIN(64); break;
-    default: return hipErrorInvalidValue;
-  }
-#undef ARK_FIN
-  return hipGetLastError();
 }
 
 hipError_t launch_adamw(uint32_t grad_dtype, const SegDesc* segs, uint32_t nseg,

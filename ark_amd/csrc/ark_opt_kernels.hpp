@@ -1,14 +1,15 @@
 // ark_opt_kernels.hpp -- gfx950 kernels of the optimizer step.
 //
-// Three stream-ordered kernels per step, no host round trip:
+// Two stream-ordered kernels per step, no host round trip:
 //   1. sumsq_kernel   : reads every gradient once (2 B/param for fp16), forms
 //                       the f64 sum of squares of the unscaled gradients along
 //                       the canonical pairwise tree and the inf/NaN flag, one
-//                       partial per block of SPB segments.
-//   2. finalize_kernel: one block; finishes the tree, runs the AMP skip /
-//                       growth state machine, the clip decision and the bias
-//                       corrections, and writes the step scalars.
-//   3. adamw_kernel   : the fused streaming update (22 B/param): unscale, clip
+//                       partial per block of SPB segments.  Its first block is
+//                       the finalizer: it takes the partials as they appear,
+//                       finishes the tree, runs the AMP skip / growth state
+//                       machine, the clip decision and the bias corrections,
+//                       and writes the step scalars.
+//   2. adamw_kernel   : the fused streaming update (22 B/param): unscale, clip
 //                       coefficient, AdamW with decoupled weight decay, fp16
 //                       weight requantisation; exits at once on a skipped step.
 //
@@ -45,7 +46,7 @@ constexpr int kRowsPerSeg = kSeg / kRow;    // 16
 constexpr uint32_t kAdamWaves = 4;          // adamw waves per block, one row each
 constexpr uint32_t kAdamStride = 32;        // rows between a block's waves
 constexpr uint32_t kAdamGroup = kAdamWaves * kAdamStride;  // rows of kAdamStride blocks
-constexpr int kFinThreads = 1024;           // finalize block
+constexpr int kFinThreads = 1024;           // clip finalize block
 
 // Segment descriptor flags.
 constexpr uint32_t kSegNoUnscale = 1u;  // ARK_OPT_TENSOR_NO_UNSCALE
@@ -63,7 +64,7 @@ struct SegDesc {
 };
 static_assert(sizeof(SegDesc) == 48, "48-byte descriptor");
 
-// Scalars of one step, written by finalize_kernel, read by adamw_kernel.
+// Scalars of one step, written by the norm pass's finalizer, read by adamw_kernel.
 struct StepScalars {
   uint32_t applied;
   uint32_t clipped;
@@ -103,37 +104,45 @@ __host__ __device__ inline float lr_eff_of(float lr, float beta1, float beta2,
 // kMaxParts partials); halved while fewer than 512 blocks would cover the
 // table.
 int sumsq_spb(uint64_t nseg, uint32_t grad_dtype);
-// Partial-buffer capacity: past kFinTarget the partials are folded by
-// kFoldGroup, so the finalize reads at most kMaxParts / kFoldGroup = 8192.
-constexpr uint32_t kMaxParts = 512u * kFinThreads;
-// Above kFinTarget partials, fold_kernel first reduces aligned groups of
-// kFoldGroup (one wave each) so the finalize reads at most kFinTarget values.
+// Group sums the norm pass's finalizer holds, and the most partials it takes
+// (64 lanes of 8 per group).
+constexpr uint32_t kFinGroups = 1024;
+constexpr uint32_t kMaxParts = kFinGroups * 64u * 8u;
+
+// What the finalizer needs (block 0 of the norm pass).  part: nparts slots,
+// every byte 0xFF before the first step; the pass leaves them so.
+struct FinalizeArgs {
+  double* part;
+  uint32_t nparts;
+  float lr;
+  const float* lr_ptr;  // NULL, or a device scalar this step's lr is read from
+  ark_opt_state* state;
+  StepScalars* scal;
+  ark_opt_step_info* info;
+  ark_opt_hparams hp;
+};
+
+// The clip's partials (launch_grad_clip): up to kFinTarget go to its finalize,
+// more are first folded in aligned groups of kFoldGroup.
 constexpr uint32_t kFinTarget = 8u * kFinThreads;
 constexpr uint32_t kFoldGroup = 64u;
-
-// in: padded_parts partials (a power of two, multiple of kFoldGroup, zero
-// past the real ones); out: padded_parts / kFoldGroup group sums.
-hipError_t launch_fold(uint32_t padded_parts, const double* in, double* out,
-                       hipStream_t stream);
 // adamw: one wave per row, 16 rows per segment; rows and work-items must stay
 // below 2^32 work-items.
 constexpr uint64_t kMaxSegments = (1ull << 32) / (64ull * kRowsPerSeg) - 1;
 static_assert((kMaxSegments + 7) / 8 <= kMaxParts, "8 segments per norm block cover every table");
-static_assert(kMaxParts / kFoldGroup <= kFinTarget, "one fold leaves the finalize kFinTarget");
 
 // ---------------------------------------------------------------------------
 // Launch helpers (ark_opt_kernels.hip); each returns hipSuccess or the error.
 // ---------------------------------------------------------------------------
 
-// part_sum: one partial per block (NaN when the block saw a non-finite
-// gradient).  A batch of segments whose segments all exist, hold kSeg
-// elements and carry kSegVec takes 16-byte loads.  Blocks b >= nt_from read
+// The norm pass, fin.nparts blocks of spb segments and the finalizer: the step's
+// scalars, state and info.  A batch of segments whose segments all exist, hold
+// kSeg elements and carry kSegVec takes 16-byte loads.  Blocks b >= nt_from read
 // with non-temporal loads (see sumsq_nt_from).  lds_bytes of dynamic LDS per
 // block (unused by the kernel) bound how many blocks a CU holds at once
 // (sumsq_lds_for).
-hipError_t launch_sumsq(uint32_t grad_dtype, int spb, uint32_t nblocks,
-                        const SegDesc* segs, uint32_t nseg, const ark_opt_state* state,
-                        double* part_sum, uint32_t nt_from, uint32_t lds_bytes,
+hipError_t launch_sumsq(uint32_t grad_dtype, int spb, const SegDesc* segs, uint32_t nseg,
+                        uint32_t nt_from, const FinalizeArgs& fin, uint32_t lds_bytes,
                         hipStream_t stream);
 
 // Resident norm blocks per CU for fp16 gradients.  Their fast path (squares
@@ -168,15 +177,8 @@ inline uint32_t sumsq_nt_from(int spb, uint64_t grad_bytes) {
   return b > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)b;
 }
 
-// Leaves per finalize thread for nparts partials (a power of two <= 64); the
-// partial buffer must hold kFinThreads * leaves doubles, zero past nparts.
+// Leaves per clip-finalize thread for nparts partials (a power of two <= 8).
 uint32_t finalize_leaves(uint32_t nparts);
-
-// lr_ptr: NULL, or a device scalar the kernel reads this step's lr from.
-hipError_t launch_finalize(uint32_t leaves, const double* part_sum,
-                           const ark_opt_hparams& hp, float lr, const float* lr_ptr,
-                           ark_opt_state* state, StepScalars* scal,
-                           ark_opt_step_info* info, hipStream_t stream);
 
 // lds_bytes: dynamic LDS per block, the residency cap (adamw_lds_for).
 hipError_t launch_adamw(uint32_t grad_dtype, const SegDesc* segs,

@@ -277,7 +277,7 @@ class Optimizer:
         return check(lib().ark_opt_step(self._h, lr, None))
 
     def step_lr_dev(self, lr_dev, info=False):
-        """One fused step whose lr the finalize kernel reads from the
+        """One fused step whose lr the norm pass reads from the
         one-element float32 GPU tensor lr_dev when it runs (graph replays
         that follow a schedule).  Returns (status, StepInfo) when info is
         True, else the status without waiting."""

@@ -128,7 +128,8 @@ typedef struct ark_opt_step_info {
 typedef struct ark_opt_timing {
   uint64_t steps;     /* steps timed                                   */
   double ms_norm;     /* total ms in the sum-of-squares / finite kernel */
-  double ms_finalize; /* total ms in the scalar finalize kernel         */
+  double ms_finalize; /* total ms from there to the AdamW pass (the norm
+                       * pass also finishes the step's scalars)         */
   double ms_adamw;    /* total ms in the fused AdamW kernel             */
   double ms_step;     /* total ms from the first to the last kernel     */
 } ark_opt_timing;
@@ -187,7 +188,7 @@ int ark_opt_destroy(ark_opt_handle *h);
 int ark_opt_step(ark_opt_handle *h, float lr, ark_opt_step_info *info);
 
 /* ark_opt_step with this step's learning rate read from the device scalar
- * *lr_dev when the step's finalize kernel runs, instead of a host value.  No
+ * *lr_dev when the step's norm pass runs, instead of a host value.  No
  * counterpart in the reference (its lr is a host value, Optimizer::lr_now,
  * optimizer.rs:80-92); for steps replayed from a HIP graph: a captured call
  * reads the scalar on every replay, so writing this step's lr into it
