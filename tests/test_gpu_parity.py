@@ -134,10 +134,26 @@ def test_norm_blocking_does_not_change_bits(grad_dtype, monkeypatch):
         opt.close()
 
 
+@pytest.mark.parametrize("grad_dtype", [_abi.GRAD_F16, _abi.GRAD_F32])
+@pytest.mark.parametrize("parts", [1, 64, 65, 256, 257, 1024, 1025, 1536, 1537, 2049])
+def test_partial_counts_around_the_finalizers_groups(parts, grad_dtype, monkeypatch):
+    """One partial per segment, on both sides of where the finalizer takes 1, 4
+    or 8 partials per lane (256, 1024) and of whole rounds and groups of 512:
+    two steps, the second finding every slot as the first left it."""
+    monkeypatch.setenv("ARK_OPT_SUMSQ_SPB", "1")
+    specs = [TensorSpec("a", (4096 * parts - 5,), True, False)]
+    cfg, ps, ts, opt, ref = _make(specs, 40 + parts, [1e-3], 2048.0, grad_dtype=grad_dtype)
+    for _ in range(2):
+        _, gi = opt.step_all(cfg.lr, info=True)
+        _, ri = ref.step(cfg.lr)
+        assert not H.info_matches(gi, ri), parts
+    opt.close()
+
+
 @pytest.mark.parametrize("cap", ["0", "4", "16", "32"])
 def test_adamw_residency_does_not_change_bits(cap, monkeypatch):
-    """Any cap on the one-wave AdamW blocks a CU holds at once (none, the
-    fewest allowed, the default, every wave slot) gives every w/m/v bit of
+    """Any cap on the AdamW waves a CU holds at once (none, the fewest
+    allowed, the default, every wave slot) gives every w/m/v bit of
     the oracle's, on ragged and unaligned tensors too."""
     monkeypatch.setenv("ARK_OPT_ADAMW_BLOCKS_PER_CU", cap)
     specs = config_tensors("c1") + [TensorSpec("r", (4096 * 5 + 3,), True, False),

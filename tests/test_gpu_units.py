@@ -84,6 +84,22 @@ def _outs(specs, seed, sigma, scale):
     return [torch.randn(s.n, device="cuda", generator=g) * (sigma * scale) for s in specs]
 
 
+@pytest.mark.parametrize("parts", [3, 1025, 2049])
+def test_partial_counts_of_the_units_finalizer(parts, monkeypatch):
+    """One partial per segment, a last block with one wave at work, and more
+    than the 1024 partials a group takes: the sums of two steps from units and
+    from the gradients."""
+    monkeypatch.setenv("ARK_OPT_SUMSQ_SPB", "1")
+    specs = [TensorSpec("a", (4096 * parts - 300,), True, False)]
+    outs = _outs(specs, parts, 1e-3, 2048.0)
+    runs = [_Run(specs, outs, 2048.0) for _ in range(2)]
+    for _ in range(2):
+        infos = [r.step(specs, fused=bool(i)) for i, r in enumerate(runs)]
+        _info_eq(*infos)
+    for r in runs:
+        r.close()
+
+
 def test_eko237m_units_step_matches_the_reading_step():
     """All 272 EKO-237M tensors (d 768: the scatter's rows are whole units),
     a 2 x 2048-token Zipf scatter, gamma_final kept scaled (the reference's
