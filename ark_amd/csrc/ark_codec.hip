@@ -143,8 +143,9 @@ int run_flat(const void* src, void* dst, uint64_t n, void* stream) {
   if (((uintptr_t)src % src_size<DIR>()) || ((uintptr_t)dst % dst_size<DIR>()))
     return ark::fail(ARK_OPT_EINVAL, "src or dst not aligned to its element");
   int rc;
-  if ((rc = ark::check_buffer(src, sb, "src", 0))) return rc;
-  if ((rc = ark::check_buffer(dst, db, "dst", 0))) return rc;
+  ark::BufferChecker checker;
+  if ((rc = checker.check(src, sb, "src", 0))) return rc;
+  if ((rc = checker.check(dst, db, "dst", 0))) return rc;
   if (overlaps(src, sb, dst, db)) return ark::fail(ARK_OPT_EINVAL, "src and dst overlap");
   {
     const void* d = dst;

@@ -6,7 +6,11 @@
 
 #include <algorithm>
 #include <atomic>
+#include <mutex>
 #include <string>
+
+// The slots' memory (StreamBuf); host code looks its address up per device.
+static __device__ __align__(256) uint8_t call_scratch[ark::kCallSlots * ark::kCallSlotBytes];
 
 namespace ark {
 
@@ -214,6 +218,117 @@ uint32_t resident_lds_bytes(const void* kernel, int threads, int blocks) {
   };
   const uint32_t a = first_at_most(blocks), z = first_at_most(blocks - 1);
   return a + (z - a) / 2;
+}
+
+namespace {
+
+constexpr int kScratchDevices = 64;
+
+struct CallSlot {
+  hipEvent_t done = nullptr;     // behind the last holder's work
+  hipStream_t last = nullptr;    // its stream, only compared
+  uint64_t stamp = 0;            // when it was given back
+  bool recorded = false, held = false;
+};
+struct CallScratch {
+  char* base = nullptr;
+  CallSlot slot[kCallSlots];
+};
+std::mutex g_call_mu;  // guards g_call and g_call_stamp
+CallScratch g_call[kScratchDevices];
+uint64_t g_call_stamp = 0;
+
+// Looks the array up and creates the events, once per device; the caller
+// holds g_call_mu.
+bool call_setup_locked(int dev) {
+  CallScratch& C = g_call[dev];
+  if (C.base) return true;
+  DeviceGuard g(dev);
+  if (!g.ok) return false;
+  void* p = nullptr;
+  if (hipGetSymbolAddress(&p, HIP_SYMBOL(call_scratch)) != hipSuccess || !p) {
+    (void)hipGetLastError();
+    return false;
+  }
+  for (CallSlot& s : C.slot) {
+    if (!s.done && hipEventCreateWithFlags(&s.done, hipEventDisableTiming) != hipSuccess) {
+      s.done = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+  }
+  C.base = (char*)p;
+  return true;
+}
+
+// Takes a slot for work on stream: one this stream used last if there is one
+// (nothing to wait for), else the longest given back.  Returns its index and
+// sets *dev and *p, or -1.
+int call_slot_take(hipStream_t stream, int* dev, void** p) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
+      (stream ? hipStreamGetDevice(stream, dev) : hipGetDevice(dev)) != hipSuccess) {
+    (void)hipGetLastError();
+    return -1;
+  }
+  if (*dev < 0 || *dev >= kScratchDevices) return -1;
+  int k = -1;
+  {
+    std::lock_guard<std::mutex> lock(g_call_mu);
+    if (!call_setup_locked(*dev)) return -1;
+    CallScratch& C = g_call[*dev];
+    for (int i = 0; i < kCallSlots; ++i) {
+      if (C.slot[i].held) continue;
+      if (C.slot[i].recorded && C.slot[i].last == stream) {
+        k = i;
+        break;
+      }
+      if (k < 0 || C.slot[i].stamp < C.slot[k].stamp) k = i;
+    }
+    if (k < 0) return -1;
+    C.slot[k].held = true;
+    *p = C.base + (size_t)k * kCallSlotBytes;
+  }
+  CallSlot& S = g_call[*dev].slot[k];  // held: this thread's alone
+  if (S.recorded && hipStreamWaitEvent(stream, S.done, 0) != hipSuccess) {
+    (void)hipGetLastError();
+    std::lock_guard<std::mutex> lock(g_call_mu);
+    S.held = false;
+    *p = nullptr;
+    return -1;
+  }
+  return k;
+}
+
+void call_slot_give(int dev, int k, hipStream_t stream) {
+  CallSlot& S = g_call[dev].slot[k];
+  if (hipEventRecord(S.done, stream) != hipSuccess) {
+    (void)hipGetLastError();
+    return;  // nothing marks the end of the queued work: the slot is not used again
+  }
+  std::lock_guard<std::mutex> lock(g_call_mu);
+  S.recorded = true;
+  S.last = stream;
+  S.stamp = ++g_call_stamp;
+  S.held = false;
+}
+
+}  // namespace
+
+hipError_t StreamBuf::alloc(size_t bytes, hipStream_t stream) {
+  s_ = stream;
+  if (bytes <= kCallSlotBytes) {
+    slot_ = call_slot_take(stream, &device_, &p);
+    if (slot_ >= 0) return hipSuccess;
+  }
+  return hipMallocAsync(&p, bytes, stream);
+}
+
+StreamBuf::~StreamBuf() {
+  if (slot_ >= 0)
+    call_slot_give(device_, slot_, s_);
+  else if (p)
+    (void)hipFreeAsync(p, s_);
 }
 
 }  // namespace ark

@@ -818,9 +818,10 @@ int scatter_check(const float* embed_grad, uint32_t vocab, uint32_t d, const uin
     return fail(ARK_OPT_EINVAL, "embed_grad, dx0 or tokens not 4-byte aligned");
   const uint64_t gbytes = (uint64_t)vocab * d * 4, xbytes = (uint64_t)batch_seq * d * 4;
   int rc;
-  if ((rc = ark::check_buffer(embed_grad, gbytes, "embed_grad", 0))) return rc;
-  if ((rc = ark::check_buffer(dx0, xbytes, "dx0", 0))) return rc;
-  if ((rc = ark::check_buffer(tokens, (uint64_t)batch_seq * 4, "tokens", 0))) return rc;
+  ark::BufferChecker checker;
+  if ((rc = checker.check(embed_grad, gbytes, "embed_grad", 0))) return rc;
+  if ((rc = checker.check(dx0, xbytes, "dx0", 0))) return rc;
+  if ((rc = checker.check(tokens, (uint64_t)batch_seq * 4, "tokens", 0))) return rc;
   if (overlaps(embed_grad, gbytes, dx0, xbytes))
     return fail(ARK_OPT_EINVAL, "embed_grad and dx0 overlap");
   return ARK_OPT_OK;
@@ -983,8 +984,9 @@ int ark_grad_accumulate(float* dst, const float* src, uint64_t n, void* stream) 
   if (((uintptr_t)dst & 3u) || ((uintptr_t)src & 3u))
     return fail(ARK_OPT_EINVAL, "dst or src not 4-byte aligned");
   int rc;
-  if ((rc = ark::check_buffer(dst, n * 4, "dst", 0))) return rc;
-  if ((rc = ark::check_buffer(src, n * 4, "src", 0))) return rc;
+  ark::BufferChecker checker;
+  if ((rc = checker.check(dst, n * 4, "dst", 0))) return rc;
+  if ((rc = checker.check(src, n * 4, "src", 0))) return rc;
   if (overlaps(dst, n * 4, src, n * 4)) return fail(ARK_OPT_EINVAL, "dst and src overlap");
   {
     const void* d = dst;
@@ -1148,7 +1150,7 @@ int ark_grad_embed_scatter(float* embed_grad, uint32_t vocab, uint32_t d, const 
   hipError_t e = ws.alloc(L.bytes, s);
   if (e != hipSuccess) {
     (void)hipGetLastError();
-    return fail(ARK_OPT_ENOMEM, "hipMallocAsync(%zu) for the scatter failed", L.bytes);
+    return fail(ARK_OPT_ENOMEM, "%zu bytes of workspace for the scatter: hipMallocAsync failed", L.bytes);
   }
   return scatter_launch(embed_grad, vocab, d, tokens, dx0, batch_seq, (char*)ws.p, L, s);
 }
@@ -1175,7 +1177,7 @@ int ark_grad_embed_scatter_final(float* embed_grad, uint32_t vocab, uint32_t d,
   hipError_t e = ws.alloc(L.bytes, U.stream);
   if (e != hipSuccess) {
     (void)hipGetLastError();
-    return fail(ARK_OPT_ENOMEM, "hipMallocAsync(%zu) for the scatter failed", L.bytes);
+    return fail(ARK_OPT_ENOMEM, "%zu bytes of workspace for the scatter: hipMallocAsync failed", L.bytes);
   }
   // the units of the rows it changes are stale from here until rewritten
   ark::opt_units_set_fresh(opt, false);

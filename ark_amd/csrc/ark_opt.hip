@@ -523,10 +523,11 @@ int ark_hip_adam_step(float* w, const float* g, float* m, float* v, uint64_t n, 
                                  {uv, uv + n * 4u, "v", 0}},
                                 {{ug, ug + n * 4u, "g", 0}})))
     return rc;
-  if ((rc = check_buffer(w, n * 4u, "w", 0))) return rc;
-  if ((rc = check_buffer(g, n * 4u, "g", 0))) return rc;
-  if ((rc = check_buffer(m, n * 4u, "m", 0))) return rc;
-  if ((rc = check_buffer(v, n * 4u, "v", 0))) return rc;
+  ark::BufferChecker checker;  // the four often lie in one allocation
+  if ((rc = checker.check(w, n * 4u, "w", 0))) return rc;
+  if ((rc = checker.check(g, n * 4u, "g", 0))) return rc;
+  if ((rc = checker.check(m, n * 4u, "m", 0))) return rc;
+  if ((rc = checker.check(v, n * 4u, "v", 0))) return rc;
   {
     const void* d[3] = {w, m, v};  // any may be another handle's gradient
     const uint64_t b[3] = {n * 4u, n * 4u, n * 4u};
@@ -560,10 +561,11 @@ int ark_hip_adam_step_f16(uint16_t* w, const float* g, float* m, float* v,
                                  {uv, uv + n * 4u, "v", 0}},
                                 {{ug, ug + n * 4u, "g", 0}})))
     return rc;
-  if ((rc = check_buffer(w, n * 2u, "w", 0))) return rc;
-  if ((rc = check_buffer(g, n * 4u, "g", 0))) return rc;
-  if ((rc = check_buffer(m, n * 4u, "m", 0))) return rc;
-  if ((rc = check_buffer(v, n * 4u, "v", 0))) return rc;
+  ark::BufferChecker checker;  // the four often lie in one allocation
+  if ((rc = checker.check(w, n * 2u, "w", 0))) return rc;
+  if ((rc = checker.check(g, n * 4u, "g", 0))) return rc;
+  if ((rc = checker.check(m, n * 4u, "m", 0))) return rc;
+  if ((rc = checker.check(v, n * 4u, "v", 0))) return rc;
   {
     const void* d[3] = {w, m, v};  // any may be another handle's gradient
     const uint64_t b[3] = {n * 2u, n * 4u, n * 4u};

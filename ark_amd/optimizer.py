@@ -22,7 +22,7 @@ from dataclasses import dataclass
 import numpy as np
 
 from . import _abi
-from ._lib import check, lib
+from ._lib import check, current_stream, lib
 
 
 @dataclass
@@ -102,7 +102,7 @@ def _single_tensor_args(w, g, m, v, w_bytes):
         raise ValueError(f"lengths differ: w {w.numel()}, g {g.numel()}, m {m.numel()}, "
                          f"v {v.numel()}")
     return (w.data_ptr(), g.data_ptr(), m.data_ptr(), v.data_ptr(), g.numel(),
-            C.c_void_p(torch.cuda.current_stream(w.device).cuda_stream))
+            current_stream(w))
 
 
 def adam_step_zero_copy(w_fp16, g, m, v, lr, beta1, beta2, eps, wd, t):
@@ -131,7 +131,7 @@ def grad_clip_global(grads, threshold, wait=True):
     import torch
     if not (grads.is_cuda and grads.is_contiguous() and grads.dtype == torch.float32):
         raise ValueError("grads must be a contiguous float32 GPU tensor")
-    st = C.c_void_p(torch.cuda.current_stream(grads.device).cuda_stream)
+    st = current_stream(grads)
     norm = C.c_float()
     check(lib().ark_hip_grad_clip(grads.data_ptr(), grads.numel(), threshold,
                                   C.byref(norm) if wait else None, st))

@@ -239,7 +239,8 @@ int ark_hip_adam_step(float *w, const float *g, float *m, float *v, uint64_t n, 
  * norm_out: a host pointer that receives the pre-clip norm (opti.s:423); the
  * call then waits for the stream, as the reference returns it.  NULL: the
  * work is only queued.  Workspace (8 bytes per 8192 values, at most
- * ~4.2 MB) comes from the stream-ordered pool; n <= 2^32. */
+ * ~4.2 MB) comes from the library's slots or the stream-ordered pool, as
+ * ark_grad_embed_scatter's; n <= 2^32. */
 int ark_hip_grad_clip(float *grads, uint64_t n, float threshold, float *norm_out, void *stream);
 
 /* Drop-in for one call of ark_asm_adam_step_f16 (opti.s:189-193, declared

@@ -159,6 +159,45 @@ def test_scatter_run_lengths_at_the_path_boundaries(d):
     np.testing.assert_array_equal(_bits(gg).reshape(vocab, d), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("threads", [1, 4])
+def test_scatter_workspaces_on_many_streams(threads):
+    """Twelve streams, more than the library keeps workspaces for, with
+    batches of different sizes queued round after round and no host wait, from
+    one thread and from four at once: every embedding gradient as the loop
+    leaves it."""
+    import threading
+    torch = _torch()
+    rng = np.random.default_rng(threads)
+    vocab, d, rounds = 500, 64, 4
+    jobs = []
+    for k in range(12):
+        n = int(rng.choice([3, 700, 4096, 13000, 40000]))
+        tokens = _zipf_tokens(rng, n, vocab)
+        dx0 = rng.standard_normal((n, d)).astype(np.float32)
+        g = rng.standard_normal((vocab, d)).astype(np.float32)
+        want = g.copy()
+        for _ in range(rounds):
+            oracle.embed_scatter(want, tokens, dx0)
+        jobs.append((torch.from_numpy(g).cuda(), torch.from_numpy(tokens.view(np.int32)).cuda(),
+                     torch.from_numpy(dx0).cuda(), want, torch.cuda.Stream()))
+    torch.cuda.synchronize()
+
+    def queue(part):
+        for _ in range(rounds):
+            for gg, tt, xx, _, stream in part:
+                with torch.cuda.stream(stream):
+                    grad.embed_scatter(gg, tt, xx)
+
+    ts = [threading.Thread(target=queue, args=(jobs[i::threads],)) for i in range(threads)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    torch.cuda.synchronize()
+    for k, (gg, _, _, want, _) in enumerate(jobs):
+        np.testing.assert_array_equal(_bits(gg).reshape(vocab, d), want.view(np.uint32), err_msg=str(k))
+
+
 @pytest.mark.parametrize("d,x_off", [(256, 0), (260, 0), (65, 0), (256, 1)])
 def test_scatter_run_lengths_around_the_block_shapes(d, x_off):
     """Runs on both sides of where one wave hands over to a block (31, 32, 33
