@@ -52,13 +52,16 @@ constexpr uint32_t kBlocksPerSeg = kSeg / (kWave * kPerLane);  // 16
 // against 443.0 us at 24 per CU, same box).
 constexpr int kPlanBlocksPerCu = 24;
 constexpr uint32_t kTileCols = 256;  // columns per wave on a short run, and per norm unit
-// run_kernel's shape.  It is bound by latency: a wave's chain is keys, rows,
-// store, and most waves find no run of theirs and leave, so what counts is how
-// many blocks are resident at once.  Measured on MI355X, 4096 Zipf tokens of
-// 768 columns (18.3 us before, plus 8.8 us for a copy of the rows in sorted
-// order): 18.6 us with 16-wave blocks (74 registers, one block per CU), 22.7 us
-// with 4-wave blocks and runs up to 64 rows left to one wave, 9.4-10.1 us as
-// here, in 62 registers.  One token at all 4096 positions: 25 us (73 us).
+// run_kernel's shape.  It is bound by latency: a wave's chain is keys,
+// positions, rows, store, and most waves find no run of theirs and leave, so
+// what counts is how many blocks are resident at once (63 registers here: four
+// blocks a CU) and how much of the longest run's chain is overlapped.  Measured
+// on MI355X, 4096 Zipf tokens of 768 columns, buffers not in cache: 9.5 us
+// (19.2 us with the rows' addresses formed one by one in the scalar unit, the
+// run's end searched for before its first rows are asked for and a sleeping
+// wait for the running sum; with 16-wave blocks or runs up to 64 rows left to
+// one wave 18-23 us; a copy of the rows in sorted order and one column per lane
+// before that 8.8 + 18.3).  One token at all 4096 positions: 23 us (73 us).
 constexpr uint32_t kLongRun = 32;  // runs of at least this many rows go to a whole block
 constexpr uint32_t kRowBatch = 8;  // rows in flight per wave on a short run
 constexpr uint32_t kRunWaves = 8;  // waves per block
@@ -556,14 +559,24 @@ __global__ __launch_bounds__(kRankWaves * kWave) void rank_sort_kernel(
 // its positions svals[start..end) increase, and its rows dx0[svals[...]] are
 // added into the key's embedding row one after the other.
 
-// Row i of dx0, by a uniform i: the base stays in scalar registers and the
-// lane adds a 32-bit byte offset (a row is below 2^26 bytes).
-template <typename T>
-__device__ __forceinline__ T ld_row(const float* dx0, uint32_t d, uint32_t i, uint32_t byte_off) {
-  uint64_t base = (uint64_t)(dx0 + (uint64_t)i * d);
-  asm("" : "+s"(base));
-  return ld_nt<T>((const char*)base + byte_off);
-}
+// The addresses of 64 rows of dx0, one per lane, formed at once; at(j) puts
+// row j's in scalar registers, to which a lane adds a 32-bit byte offset (a row
+// is below 2^26 bytes).
+struct RowAddr {
+  uint32_t lo, hi;
+  __device__ __forceinline__ RowAddr(const float* dx0, uint32_t d, uint32_t row) {
+    const uint64_t a = (uint64_t)(dx0 + (uint64_t)row * d);
+    lo = (uint32_t)a;
+    hi = (uint32_t)(a >> 32);
+  }
+  template <typename T>
+  __device__ __forceinline__ T load(uint32_t j, uint32_t byte_off) const {
+    uint64_t a = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, j) << 32 |
+                 (uint32_t)__builtin_amdgcn_readlane(lo, j);
+    asm("" : "+s"(a));
+    return ld_nt<T>((const char*)a + byte_off);
+  }
+};
 
 // A run shorter than kLongRun that starts at sorted position p, columns
 // [256 * tile, +256) of the row, by one wave.  Rows are loaded kRowBatch at a
@@ -585,6 +598,7 @@ __device__ __forceinline__ void short_run(float* __restrict__ g, uint32_t d,
   const uint64_t other = ~__ballot(k == t && p + lane < n && lane < kLongRun);
   const uint32_t len = (uint32_t)__ffsll((unsigned long long)other) - 1u;
   if (len == kLongRun) return;  // long_run's
+  const RowAddr rows(dx0, d, pos);
   const uint32_t c0 = tile * kTileCols;
   if constexpr (VEC) {
     const uint32_t c = c0 + 4u * lane, cl = c < d ? c : d - 4u;  // past d: loaded, not stored
@@ -595,7 +609,7 @@ __device__ __forceinline__ void short_run(float* __restrict__ g, uint32_t d,
 #pragma unroll
       for (uint32_t j = 0; j < kRowBatch; ++j)
         if (b + j < len)
-          v[j] = ld_row<f32x4>(dx0, d, __builtin_amdgcn_readlane(pos, b + j), cl * 4u);
+          v[j] = rows.load<f32x4>(b + j, cl * 4u);
 #pragma unroll
       for (uint32_t j = 0; j < kRowBatch; ++j) {
         if (b + j < len) {
@@ -621,10 +635,9 @@ __device__ __forceinline__ void short_run(float* __restrict__ g, uint32_t d,
 #pragma unroll
       for (uint32_t j = 0; j < kRowBatch; ++j) {
         if (b + j < len) {
-          const uint32_t i = __builtin_amdgcn_readlane(pos, b + j);
 #pragma unroll
           for (int u = 0; u < 4; ++u)
-            v[j][u] = ld_row<float>(dx0, d, i, (c[u] < d ? c[u] : d - 1u) * 4u);
+            v[j][u] = rows.load<float>(b + j, (c[u] < d ? c[u] : d - 1u) * 4u);
         }
       }
 #pragma unroll
@@ -644,16 +657,17 @@ __device__ __forceinline__ void short_run(float* __restrict__ g, uint32_t d,
 // The run that holds sorted position p (a multiple of kLongRun), columns
 // [64 * ctile, +64), by the whole block: lane l of every wave owns column l.
 // Chunk c of the run is its rows [c * kColRows, +kColRows); wave w loads the
-// chunks w, w + kRunWaves, ... into registers ahead of their turn, and the running
-// sum goes from chunk to chunk through LDS, so up to kRunWaves * kColRows rows are in
-// flight while the additions keep the run's order.  A run of kLongRun rows
-// covers a multiple of kLongRun; the block at the first one takes the run.
+// chunks w, w + kRunWaves, ... into registers ahead of their turn, and the
+// running sum goes from chunk to chunk through LDS, so up to kRunWaves *
+// kColRows rows are in flight while the additions keep the run's order.  A lane
+// passes its sum and the chunk number on in one 64-bit word, so taking over
+// costs one LDS read.  A run of kLongRun rows covers a multiple of kLongRun; the
+// block at the first one takes the run.
 __device__ __forceinline__ void long_run(float* __restrict__ g, uint32_t d,
                                          const float* __restrict__ dx0,
                                          const uint32_t* __restrict__ skeys,
                                          const uint32_t* __restrict__ svals, uint32_t n,
-                                         uint32_t p, uint32_t ctile, float* s_acc,
-                                         uint32_t* s_turn) {
+                                         uint32_t p, uint32_t ctile, uint64_t* s_sum) {
   const uint32_t lane = __lane_id();
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   // the kWave keys from p on, and those before it
@@ -666,9 +680,27 @@ __device__ __forceinline__ void long_run(float* __restrict__ g, uint32_t d,
   const uint32_t ahead = fwd ? (uint32_t)__ffsll((unsigned long long)fwd) - 1u : kWave;
   if (back == kLongRun || back + ahead < kLongRun) return;  // an earlier block's, or short
   const uint32_t start = p - back;
-  uint32_t end = p + ahead;
+  const uint32_t c = ctile * kWave + lane;
+  const uint32_t cl = c < d ? c : d - 1u;  // lanes past d load the last column
+  uint32_t end = fwd ? p + ahead : n;      // until the search below: at most
+  // a chunk's positions, one per lane, and its rows; past the end, the last one
+  auto positions = [&](uint32_t ch) {
+    const uint32_t k = start + ch * kColRows + lane;
+    return ld_g<uint32_t>(svals + (k < end ? k : end - 1u));
+  };
+  float v[kColRows];
+  auto load_rows = [&](uint32_t pos) {
+    const RowAddr rows(dx0, d, pos);
+#pragma unroll
+    for (uint32_t j = 0; j < kColRows; ++j) v[j] = rows.load<float>(j, cl * 4u);
+  };
+  uint32_t next = positions(wave);
+  if (wave == 0) s_sum[lane] = 0ull;  // no chunk done
+  __syncthreads();
+  if (start + wave * kColRows < end) load_rows(next);
   if (!fwd) {
-    // skeys[lo] == t and skeys[hi] != t (or hi == n), narrowed kWave probes at a time
+    // The end, while the first rows are on their way: skeys[lo] == t and
+    // skeys[hi] != t (or hi == n), narrowed kWave probes at a time.
     uint32_t lo = p + kWave - 1u, hi = n;
     while (hi - lo > 1u) {
       const uint32_t step = (hi - lo + kWave - 1u) / kWave;
@@ -681,39 +713,21 @@ __device__ __forceinline__ void long_run(float* __restrict__ g, uint32_t d,
     }
     end = hi;
   }
-  if (threadIdx.x == 0) *s_turn = 0u;
-  __syncthreads();
-  const uint32_t c = ctile * kWave + lane;
-  const uint32_t cl = c < d ? c : d - 1u;  // lanes past d load the last column
   const uint32_t chunks = (end - start + kColRows - 1u) / kColRows;
-  auto positions = [&](uint32_t ch) {  // chunk ch's, one per lane; past the run, its last
-    const uint32_t k = start + ch * kColRows + lane;
-    return ld_g<uint32_t>(svals + (k < end ? k : end - 1u));
-  };
-  uint32_t next = positions(wave);
   for (uint32_t ch = wave; ch < chunks; ch += kRunWaves) {
     const uint32_t k0 = start + ch * kColRows;
     const uint32_t cnt = end - k0 < kColRows ? end - k0 : kColRows;
-    const uint32_t pos = next;
-    float v[kColRows];
-    if (cnt == kColRows) {
-#pragma unroll
-      for (uint32_t j = 0; j < kColRows; ++j)
-        v[j] = ld_row<float>(dx0, d, __builtin_amdgcn_readlane(pos, j), cl * 4u);
-    } else {
-#pragma unroll
-      for (uint32_t j = 0; j < kColRows; ++j)
-        if (j < cnt)
-          v[j] = ld_row<float>(dx0, d, __builtin_amdgcn_readlane(pos, j), cl * 4u);
-    }
+    if (ch != wave) load_rows(next);
     next = positions(ch + kRunWaves);  // in flight while the wave waits its turn
     float acc;
     if (ch == 0u) {
       acc = ld_g<float>(g + (uint64_t)t * d + cl);
     } else {
-      while (__hip_atomic_load(s_turn, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) != ch)
-        __builtin_amdgcn_s_sleep(1);
-      acc = s_acc[lane];
+      uint64_t x;
+      do {
+        x = __hip_atomic_load(s_sum + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      } while (!__all((uint32_t)(x >> 32) == ch));
+      acc = __uint_as_float((uint32_t)x);
     }
     if (cnt == kColRows) {
 #pragma unroll
@@ -726,9 +740,8 @@ __device__ __forceinline__ void long_run(float* __restrict__ g, uint32_t d,
     if (ch + 1u == chunks) {
       if (c < d) st_g<float>(g + (uint64_t)t * d + c, acc);
     } else {
-      s_acc[lane] = acc;
-      if (lane == 0)
-        __hip_atomic_store(s_turn, ch + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __hip_atomic_store(s_sum + lane, (uint64_t)(ch + 1u) << 32 | __float_as_uint(acc),
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
   }
 }
@@ -743,12 +756,11 @@ __global__ __launch_bounds__(kRunWaves * kWave) void run_kernel(
     float* __restrict__ g, uint32_t d, const float* __restrict__ dx0,
     const uint32_t* __restrict__ skeys, const uint32_t* __restrict__ svals,
     uint32_t n, uint32_t p0, uint32_t p1, uint32_t nlong) {
-  __shared__ float s_acc[kWave];
-  __shared__ uint32_t s_turn;
+  __shared__ uint64_t s_sum[kWave];
   if (blockIdx.x < nlong) {
     const uint32_t ctiles = (d + kWave - 1u) / kWave;
     long_run(g, d, dx0, skeys, svals, n, p0 + blockIdx.x / ctiles * kLongRun,
-             blockIdx.x % ctiles, s_acc, &s_turn);
+             blockIdx.x % ctiles, s_sum);
     return;
   }
   const uint32_t tiles = (d + kTileCols - 1u) / kTileCols;
