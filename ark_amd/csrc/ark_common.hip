@@ -228,6 +228,7 @@ struct CallSlot {
   hipEvent_t done = nullptr;     // behind the last holder's work
   hipStream_t last = nullptr;    // its stream, only compared
   uint64_t stamp = 0;            // when it was given back
+  float* host = nullptr;         // pinned, allocated when first asked for
   bool recorded = false, held = false;
 };
 struct CallScratch {
@@ -322,6 +323,20 @@ hipError_t StreamBuf::alloc(size_t bytes, hipStream_t stream) {
     if (slot_ >= 0) return hipSuccess;
   }
   return hipMallocAsync(&p, bytes, stream);
+}
+
+float* StreamBuf::host() {
+  if (slot_ < 0) return nullptr;
+  CallSlot& S = g_call[device_].slot[slot_];  // held: this thread's alone
+  if (!S.host) {
+    void* p = nullptr;
+    if (hipHostMalloc(&p, 64, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    S.host = (float*)p;
+  }
+  return S.host;
 }
 
 StreamBuf::~StreamBuf() {

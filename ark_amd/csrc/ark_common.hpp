@@ -131,6 +131,9 @@ class StreamBuf {
  public:
   void* p = nullptr;
   hipError_t alloc(size_t bytes, hipStream_t stream);
+  // A float of pinned host memory that goes with the slot, for a kernel to
+  // answer the waiting caller in; NULL when the memory is not a slot's.
+  float* host();
   ~StreamBuf();
 
  private:

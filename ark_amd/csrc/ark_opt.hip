@@ -68,8 +68,7 @@ struct ark_opt_handle {
   double* d_part_sum = nullptr;  // one slot per norm block
   ark_opt_state* d_state = nullptr;
   StepScalars* d_scal = nullptr;
-  ark_opt_step_info* d_info = nullptr;
-  ark_opt_step_info* h_info = nullptr;  // pinned
+  ark_opt_step_info* h_info = nullptr;  // pinned, written by the step's kernels when asked for
   ark_opt_state* h_state = nullptr;     // pinned
   // the norm's units (fp32-gradient handles): written by the gradient
   // producers' final kernels, consumed by the next step instead of the read
@@ -310,8 +309,6 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
   off = align_up(off + sizeof(ark_opt_state), 256);
   const size_t o_scal = off;
   off = align_up(off + sizeof(StepScalars), 256);
-  const size_t o_info = off;
-  off = align_up(off + sizeof(ark_opt_step_info), 256);
   const size_t o_units = off;
   if (hp->grad_dtype == ARK_OPT_GRAD_F32)
     off = align_up(off + sizeof(double) * (size_t)nseg * ark::kUnitsPerSeg, 256);
@@ -327,7 +324,6 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
   h->d_part_sum = (double*)(base + o_psum);
   h->d_state = (ark_opt_state*)(base + o_state);
   h->d_scal = (StepScalars*)(base + o_scal);
-  h->d_info = (ark_opt_step_info*)(base + o_info);
   if (hp->grad_dtype == ARK_OPT_GRAD_F32 && nseg) h->d_units = (double*)(base + o_units);
   {
     uint64_t seg0 = 0;
@@ -370,8 +366,6 @@ int ark_opt_destroy(ark_opt_handle* h) {
 }
 
 static int finish_info(ark_opt_handle* h, ark_opt_step_info* info) {
-  ARK_HIP(hipMemcpyAsync(h->h_info, h->d_info, sizeof(ark_opt_step_info),
-                         hipMemcpyDeviceToHost, h->stream));
   ARK_HIP(hipStreamSynchronize(h->stream));
   *info = *h->h_info;
   return info->status;
@@ -400,7 +394,7 @@ int step_impl(ark_opt_handle* h, float lr, const float* lr_dev, ark_opt_step_inf
   fin.lr_ptr = lr_dev;
   fin.state = h->d_state;
   fin.scal = h->d_scal;
-  fin.info = h->d_info;
+  fin.host_info = info ? h->h_info : nullptr;
   fin.hp = h->hp;
   if (take_fresh_units(h)) {
     // the gradients' producers already formed the tree's first level
@@ -453,7 +447,8 @@ int ark_opt_record_overflow(ark_opt_handle* h, ark_opt_step_info* info) {
   DeviceGuard g(h->device);
   if (!g.ok) return fail(ARK_OPT_EHIP, "cannot select device %d", h->device);
   ark::opt_units_set_fresh(h, false);  // the loss scale they were unscaled by changes
-  ARK_HIP(ark::launch_record_overflow(h->hp, h->d_state, h->d_info, h->stream));
+  ARK_HIP(ark::launch_record_overflow(h->hp, h->d_state, info ? h->h_info : nullptr,
+                                       h->stream));
   if (info) return finish_info(h, info);
   return ARK_OPT_OK;
 }
@@ -604,23 +599,24 @@ int ark_hip_grad_clip(float* grads, uint64_t n, float threshold, float* norm_out
   hipStream_t s = (hipStream_t)stream;
   const uint32_t nparts = ark::clip_parts(n);
   const uint32_t ngroups = (nparts + ark::kFoldGroup - 1) / ark::kFoldGroup;
-  const size_t bytes = ark::align_up(sizeof(ark::ClipScalars), 256) +
-                       ark::align_up((size_t)nparts * 8u, 256) + (size_t)ngroups * 8u;
+  const size_t parts_bytes = ark::align_up((size_t)nparts * 8u, 256);
+  const size_t bytes = 256 + parts_bytes + (size_t)ngroups * 8u;
   ark::StreamBuf ws;
   hipError_t e = ws.alloc(bytes, s);
   if (e != hipSuccess) {
     (void)hipGetLastError();
-    return fail(ARK_OPT_ENOMEM, "hipMallocAsync(%zu) for the clip failed", bytes);
+    return fail(ARK_OPT_ENOMEM, "%zu bytes of workspace for the clip: hipMallocAsync failed", bytes);
   }
-  ark::ClipScalars* cs = (ark::ClipScalars*)ws.p;
-  double* parts = (double*)((char*)ws.p + ark::align_up(sizeof(ark::ClipScalars), 256));
-  double* folded = parts + ark::align_up((size_t)nparts * 8u, 256) / 8u;
-  ARK_HIP(ark::launch_grad_clip(grads, n, threshold, parts, folded, cs, s));
+  float* norm = (float*)ws.p;
+  double* parts = (double*)((char*)ws.p + 256);
+  double* folded = parts + parts_bytes / 8u;
+  float* host_norm = norm_out ? ws.host() : nullptr;
+  ARK_HIP(ark::launch_grad_clip(grads, n, threshold, parts, folded, host_norm ? host_norm : norm, s));
   if (norm_out) {
-    float norm = 0.0f;
-    ARK_HIP(hipMemcpyAsync(&norm, &cs->norm, sizeof(float), hipMemcpyDeviceToHost, s));
+    float x = 0.0f;
+    if (!host_norm) ARK_HIP(hipMemcpyAsync(&x, norm, sizeof(float), hipMemcpyDeviceToHost, s));
     ARK_HIP(hipStreamSynchronize(s));
-    *norm_out = norm;
+    *norm_out = host_norm ? *host_norm : x;
   }
   return ARK_OPT_OK;
 }

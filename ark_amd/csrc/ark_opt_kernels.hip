@@ -364,7 +364,7 @@ __device__ __forceinline__ void finalize_step(const FinalizeArgs& a, double* sum
   out.state = st;
   *a.state = st;
   *a.scal = sc;
-  *a.info = out;
+  if (a.host_info) *a.host_info = out;
 }
 
 // ---- kernel 1: sum of squares + non-finite flag -----------------------------
@@ -575,7 +575,7 @@ __global__ __launch_bounds__(kBlock) void units_reduce_kernel(const double* __re
 
 __global__ void record_overflow_kernel(ark_opt_hparams hp,
                                        ark_opt_state* __restrict__ state,
-                                       ark_opt_step_info* __restrict__ info) {
+                                       ark_opt_step_info* __restrict__ host_info) {
   ark_opt_state st = *state;
   ark_opt_step_info out = {};
   out.nonfinite = 1;
@@ -588,7 +588,7 @@ __global__ void record_overflow_kernel(ark_opt_hparams hp,
   }
   out.state = st;
   *state = st;
-  *info = out;
+  if (host_info) *host_info = out;
 }
 
 // ---- kernel 3: fused AdamW -------------------------------------------------
@@ -862,63 +862,46 @@ __global__ __launch_bounds__(kFoldGroup) void clip_fold_kernel(const double* __r
   if (threadIdx.x == 0) out[blockIdx.x] = x;
 }
 
-// The root of the tree over nparts leaves (zero past them, padded to
-// kFinThreads * L), as finalize_kernel forms it; then the decision of
-// opti.s:399-404: norm = fsqrt of the sum as fp32 (the reference's sum is
-// fp32), clipped when norm > threshold (fcmp + b.le: an unordered compare
-// does not clip), coefficient threshold / norm.
+// Every block forms the root of the tree over nparts leaves (zero past them,
+// padded to kBlock * L) and takes the decision of opti.s:399-404 for itself, norm =
+// fsqrt of the sum as fp32 (the reference's sum is fp32), clipped when norm >
+// threshold (fcmp + b.le: an unordered compare does not clip), coefficient
+// threshold / norm; then g[i] = g[i] * coef (fmul, opti.s:409-420) over its share,
+// grid-stride over 4-element groups, or nothing.  Block 0 reports the norm.  The
+// leaves (24 KB for 24.6M values) come from the L2s in about the time a launch
+// of its own for the decision took to start (3.9 us and a gap on MI355X).
 template <int L>
-__global__ __launch_bounds__(kFinThreads) void clip_finalize_kernel(
-    const double* __restrict__ leaves, uint32_t nparts, float threshold,
-    ClipScalars* __restrict__ out) {
-  __shared__ double wsum[kFinThreads / 64];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
+__global__ __launch_bounds__(kBlock) void clip_scale_kernel(
+    float* __restrict__ g, uint64_t n, uint32_t vec, const double* __restrict__ leaves,
+    uint32_t nparts, float threshold, float* __restrict__ norm_out) {
+  __shared__ double wsum[kBlock / 64];
+  const uint32_t tid = threadIdx.x;
   double q[L];
 #pragma unroll
   for (int j = 0; j < L; ++j) {
-    const uint32_t i = (uint32_t)tid * L + j;
+    const uint32_t i = tid * L + j;
     q[j] = i < nparts ? leaves[i] : 0.0;
   }
 #pragma unroll
   for (int w = L / 2; w >= 1; w /= 2)
 #pragma unroll
     for (int j = 0; j < w; ++j) q[j] = q[2 * j] + q[2 * j + 1];
-  double x = butterfly_from<0>(q[0]);
-  if (lane == 0) wsum[wave] = x;
+  const double x = butterfly_from<0>(q[0]);
+  if ((tid & 63u) == 0u) wsum[tid >> 6] = x;
   __syncthreads();
-  if (wave != 0) return;
-  double y = lane < kFinThreads / 64 ? wsum[lane] : 0.0;
-#pragma unroll
-  for (int s = 0; s < log2i(kFinThreads / 64); ++s) y = y + __shfl_xor(y, 1 << s);
-  if (lane != 0) return;
-  ClipScalars c;
-  c.sumsq = y;
-  c.norm = sqrtf((float)y);
-  c.clipped = c.norm > threshold ? 1u : 0u;
-  c.coef = c.clipped ? threshold / c.norm : 1.0f;
-  *out = c;
-}
-
-// g[i] = g[i] * coef (fmul, opti.s:409-420) when the finalize decided to
-// clip; otherwise every block exits at once.  Grid-stride over 4-element
-// groups.
-__global__ __launch_bounds__(256) void clip_scale_kernel(float* __restrict__ g, uint64_t n,
-                                                         uint32_t vec,
-                                                         const ClipScalars* __restrict__ cs) {
-  const uint32_t clipped = cs->clipped;
-  const float coef = cs->coef;
-  if (!clipped) return;
-  const uint64_t stride = (uint64_t)gridDim.x * 256u * 4u;
-  for (uint64_t e = ((uint64_t)blockIdx.x * 256u + threadIdx.x) * 4u; e < n; e += stride) {
+  const float norm = sqrtf((float)((wsum[0] + wsum[1]) + (wsum[2] + wsum[3])));
+  if (blockIdx.x == 0 && tid == 0) *norm_out = norm;
+  if (!(norm > threshold)) return;
+  const float coef = threshold / norm;
+  const uint64_t stride = (uint64_t)gridDim.x * kBlock * 4u;
+  for (uint64_t e = ((uint64_t)blockIdx.x * kBlock + tid) * 4u; e < n; e += stride) {
     if (vec && e + 4u <= n) {
-      f32x4 x = ld_nt<f32x4>(g + e);
-      x.x = x.x * coef;
-      x.y = x.y * coef;
-      x.z = x.z * coef;
-      x.w = x.w * coef;
-      st_nt<f32x4>(g + e, x);
+      f32x4 y = ld_nt<f32x4>(g + e);
+      y.x = y.x * coef;
+      y.y = y.y * coef;
+      y.z = y.z * coef;
+      y.w = y.w * coef;
+      st_nt<f32x4>(g + e, y);
     } else {
       for (uint64_t j = e; j < e + 4u && j < n; ++j) st_g<float>(g + j, ld_g<float>(g + j) * coef);
     }
@@ -928,7 +911,7 @@ __global__ __launch_bounds__(256) void clip_scale_kernel(float* __restrict__ g, 
 }  // namespace
 
 hipError_t launch_grad_clip(float* g, uint64_t n, float threshold, double* parts,
-                            double* folded, ClipScalars* out, hipStream_t stream) {
+                            double* folded, float* norm, hipStream_t stream) {
   const uint32_t nparts = clip_parts(n);
   const uint32_t vec = ((uintptr_t)g & 15u) == 0 ? 1u : 0u;
   const uint32_t nt_from = (uint32_t)(kNormCachedBytes / (2u * kSeg * sizeof(float)));
@@ -946,21 +929,21 @@ hipError_t launch_grad_clip(float* g, uint64_t n, float threshold, double* parts
     leaves = folded;
     nleaves = groups;
   }
-  const dim3 one(1), fin(kFinThreads);
-#define ARK_CLIP_FIN(L)                                                                         hipLaunchKernelGGL((clip_finalize_kernel<L>), one, fin, 0, stream, leaves, nleaves, threshold,                      out)
-  switch (finalize_leaves(nleaves)) {
-    case 1: ARK_CLIP_FIN(1); break;
-    case 2: ARK_CLIP_FIN(2); break;
-    case 4: ARK_CLIP_FIN(4); break;
-    case 8: ARK_CLIP_FIN(8); break;
-    default: return hipErrorInvalidValue;
-  }
-#undef ARK_CLIP_FIN
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  uint64_t blocks = (n + 1023u) / 1024u;
-  if (blocks > 65536u) blocks = 65536u;
-  hipLaunchKernelGGL(clip_scale_kernel, dim3((uint32_t)blocks), dim3(256), 0, stream, g, n, vec,
-                     (const ClipScalars*)out);
+  uint64_t blocks = (n + 4u * kBlock - 1u) / (4u * kBlock);
+  if (blocks > kClipBlocks) blocks = kClipBlocks;
+  const dim3 grid((uint32_t)blocks), block(kBlock);
+#define ARK_CLIP(L)                                                                        \
+  hipLaunchKernelGGL((clip_scale_kernel<L>), grid, block, 0, stream, g, n, vec, leaves, nleaves, \
+                     threshold, norm)
+  if (nleaves <= kBlock)
+    ARK_CLIP(1);
+  else if (nleaves <= 4u * kBlock)
+    ARK_CLIP(4);
+  else if (nleaves <= 16u * kBlock)
+    ARK_CLIP(16);
+  else
+    ARK_CLIP(32);
+#undef ARK_CLIP
   return hipGetLastError();
 }
 
@@ -1044,12 +1027,6 @@ uint32_t adamw_lds_for(uint32_t grad_dtype, int waves) {
   return resident_lds_bytes(k, 64 * kAdamWaves, (waves + kAdamWaves - 1) / kAdamWaves);
 }
 
-uint32_t finalize_leaves(uint32_t nparts) {
-  uint32_t L = 1;
-  while ((uint64_t)L * kFinThreads < nparts) L <<= 1;
-  return L;
-}
-
 hipError_t launch_adamw(uint32_t grad_dtype, const SegDesc* segs, uint32_t nseg,
                         const StepScalars* scal, float beta1, float beta2,
                         float eps, uint32_t lds_bytes, hipStream_t stream) {
@@ -1098,9 +1075,9 @@ hipError_t launch_adamw_single_w32(float* w, const float* g, float* m, float* v,
 
 hipError_t launch_record_overflow(const ark_opt_hparams& hp,
                                   ark_opt_state* state,
-                                  ark_opt_step_info* info, hipStream_t stream) {
+                                  ark_opt_step_info* host_info, hipStream_t stream) {
   hipLaunchKernelGGL(record_overflow_kernel, dim3(1), dim3(1), 0, stream, hp,
-                     state, info);
+                     state, host_info);
   return hipGetLastError();
 }
 

@@ -46,7 +46,6 @@ constexpr int kRowsPerSeg = kSeg / kRow;    // 16
 constexpr uint32_t kAdamWaves = 4;          // adamw waves per block, one row each
 constexpr uint32_t kAdamStride = 32;        // rows between a block's waves
 constexpr uint32_t kAdamGroup = kAdamWaves * kAdamStride;  // rows of kAdamStride blocks
-constexpr int kFinThreads = 1024;           // clip finalize block
 
 // Segment descriptor flags.
 constexpr uint32_t kSegNoUnscale = 1u;  // ARK_OPT_TENSOR_NO_UNSCALE
@@ -118,13 +117,13 @@ struct FinalizeArgs {
   const float* lr_ptr;  // NULL, or a device scalar this step's lr is read from
   ark_opt_state* state;
   StepScalars* scal;
-  ark_opt_step_info* info;
+  ark_opt_step_info* host_info;  // NULL, or pinned host memory that gets the step's info
   ark_opt_hparams hp;
 };
 
-// The clip's partials (launch_grad_clip): up to kFinTarget go to its finalize,
-// more are first folded in aligned groups of kFoldGroup.
-constexpr uint32_t kFinTarget = 8u * kFinThreads;
+// The clip's partials (launch_grad_clip): up to kFinTarget are taken as they
+// are, more are first folded in aligned groups of kFoldGroup.
+constexpr uint32_t kFinTarget = 8192u;
 constexpr uint32_t kFoldGroup = 64u;
 // adamw: one wave per row, 16 rows per segment; rows and work-items must stay
 // below 2^32 work-items.
@@ -177,9 +176,6 @@ inline uint32_t sumsq_nt_from(int spb, uint64_t grad_bytes) {
   return b > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)b;
 }
 
-// Leaves per clip-finalize thread for nparts partials (a power of two <= 8).
-uint32_t finalize_leaves(uint32_t nparts);
-
 // lds_bytes: dynamic LDS per block, the residency cap (adamw_lds_for).
 hipError_t launch_adamw(uint32_t grad_dtype, const SegDesc* segs,
                         uint32_t nseg, const StepScalars* scal, float beta1,
@@ -201,28 +197,24 @@ hipError_t launch_adamw_single_w32(float* w, const float* g, float* m, float* v,
 
 // The single-tensor clip (ark_asm_grad_clip, opti.s:369-432): the
 // canonical tree's sum of squares of one fp32 array (one partial per block of
-// two segments, folded past kFinTarget partials), the norm and the clip
-// decision on the device, then the in-place scaling when it clips.
-struct ClipScalars {
-  double sumsq;
-  float norm;      // the pre-clip norm the call reports
-  float coef;      // threshold / norm (1 when not clipped)
-  uint32_t clipped;
-  uint32_t pad;
-};
-static_assert(sizeof(ClipScalars) == 24, "24-byte clip result");
-// Elements one call takes: the partials stay within what one fold and a
-// 1024 x 8-leaf finalize reduce (kFinTarget * kFoldGroup = 2^19 blocks of
-// 2 segments).
+// two segments, folded past kFinTarget partials), then the norm, the clip
+// decision and the in-place scaling.
+//
+// Elements one call takes: the partials stay within what one fold leaves
+// kFinTarget of (2^19 blocks of 2 segments).
 constexpr uint64_t kClipMaxElements = (uint64_t)kFinTarget * kFoldGroup * 2u * kSeg;
 inline uint32_t clip_parts(uint64_t n) { return (uint32_t)((n + 2u * kSeg - 1) / (2u * kSeg)); }
+// Most blocks of the scaling launch, each of which forms the decision: all of
+// them resident at once.
+constexpr uint64_t kClipBlocks = 2048;
 // parts: clip_parts(n) doubles; folded: ceil(clip_parts(n) / kFoldGroup)
-// doubles (used past kFinTarget partials); out: the decision.  n >= 1.
+// doubles (used past kFinTarget partials); norm: device-visible, gets the
+// pre-clip norm.  n >= 1.
 hipError_t launch_grad_clip(float* g, uint64_t n, float threshold, double* parts,
-                            double* folded, ClipScalars* out, hipStream_t stream);
+                            double* folded, float* norm, hipStream_t stream);
 
 hipError_t launch_record_overflow(const ark_opt_hparams& hp,
                                   ark_opt_state* state,
-                                  ark_opt_step_info* info, hipStream_t stream);
+                                  ark_opt_step_info* host_info, hipStream_t stream);
 
 }  // namespace ark
