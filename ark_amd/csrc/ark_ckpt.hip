@@ -14,7 +14,8 @@
 //                 uniform misalignment.  Chunks that straddle a tensor's
 //                 edge, or whose second block would pass the end of the
 //                 source, go byte by byte.
-//   header_kernel the file header, tensor headers and trailer, byte stores.
+//                 Its last blocks write the file header, tensor headers and
+//                 trailer, byte stores.
 //   unpack_kernel one block per 2048 (fp16) or 1024 (fp32) elements of one
 //                 tensor (found the same way, both file types in one
 //                 launch); a lane takes
@@ -52,7 +53,7 @@ constexpr uint64_t kFileHeaderV4 = 28;  // u32 magic + 3 x u64 (io.rs:453-456)
 constexpr uint64_t kRecHeaderV4 = 16;   // u64 n + u64 type (io.rs:460-461, :467-468)
 constexpr uint64_t kTrailerBytes = 40;  // u32 magic + u32 version + ark_opt_state
 constexpr uint32_t kTrailerVersion = 1;
-constexpr int kThreads = 256;  // header and check kernels
+constexpr int kThreads = 256;  // check kernel
 constexpr uint32_t kHintShift = 8;  // pack/unpack blocks per find_rec hint: 256
 // Pack and unpack launch shapes: lanes per block, and 16-byte image chunks
 // (pack) or units (unpack) per lane, kLanes * 16 bytes apart.  Measured on
@@ -90,7 +91,7 @@ inline uint64_t esize(uint32_t t) { return t == ARK_CKPT_F16 ? 2u : 4u; }
 
 // The bytes of a V4 image that change from one save of the same records to
 // the next: the file header (global step, Adam step, record count) and the
-// AMP trailer.  Passed to the header kernel by value, so a prepared table
+// AMP trailer.  Passed to the pack kernel by value, so a prepared table
 // (ark_ckpt_plan) needs no upload per save.
 constexpr uint32_t kDynBytes = (uint32_t)(kFileHeaderV4 + kTrailerBytes);
 struct DynHdr {
@@ -130,6 +131,7 @@ struct UnpackRec {
 };
 static_assert(sizeof(UnpackRec) == 32, "32-byte descriptor");
 
+constexpr uint32_t kNoFailure = 0xFFFFFFFFu;
 struct CheckDesc {  // expected tensor header at an image offset
   uint64_t hdr_off;
   uint64_t n;
@@ -165,10 +167,9 @@ __device__ __forceinline__ void st_u8(uint8_t* p, uint32_t v) { st_g<uint8_t>(p,
 // thread npieces the file header and, when the image has one, the trailer,
 // from dyn (unrolled, so every byte is read from the kernel arguments at a
 // fixed offset).
-__global__ __launch_bounds__(kThreads) void header_kernel(const HdrPiece* __restrict__ pieces,
-                                                          uint32_t npieces, DynHdr dyn,
-                                                          uint8_t* __restrict__ img) {
-  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+__device__ __forceinline__ void write_header(uint32_t i, const HdrPiece* __restrict__ pieces,
+                                             uint32_t npieces, const DynHdr& dyn,
+                                             uint8_t* __restrict__ img) {
   if (i < npieces) {
     const HdrPiece* p = pieces + i;
     const uint64_t off = p->off;
@@ -205,12 +206,20 @@ __device__ __forceinline__ uint32_t find_rec(const uint32_t* __restrict__ start,
 }
 
 // Block j of a tensor covers image bytes [base + j*S, base + (j+1)*S) of its
-// data, base = data_off rounded down to 16, clipped to the data.
+// data, base = data_off rounded down to 16, clipped to the data.  Blocks from
+// nblocks up write the headers (a launch of their own for them cost 3 us and
+// the gap before it, as much as a small model's data).
 __global__ __launch_bounds__(kPackLanes) void pack_kernel(const PackRec* __restrict__ recs,
                                                           const uint32_t* __restrict__ start,
                                                           const uint32_t* __restrict__ hint,
                                                           uint8_t* __restrict__ img,
-                                                          uint32_t block0) {
+                                                          uint32_t block0, uint32_t nblocks,
+                                                          const HdrPiece* __restrict__ pieces,
+                                                          uint32_t npieces, DynHdr dyn) {
+  if (blockIdx.x >= nblocks) {
+    write_header((blockIdx.x - nblocks) * kPackLanes + threadIdx.x, pieces, npieces, dyn, img);
+    return;
+  }
   const uint32_t blk = block0 + blockIdx.x;
   const uint32_t r = find_rec(start, hint, blk);
   const PackRec s = recs[r];
@@ -346,13 +355,21 @@ __device__ __forceinline__ void unpack_block(const UnpackRec& s, uint64_t e_begi
 }
 
 // Block j of a tensor converts its elements [j*S, (j+1)*S), S = unpack_seg of
-// the tensor's file type.
+// the tensor's file type; blocks [0, blocks) hold data.  Nothing is written
+// when check_kernel left an index in *bad; the first block passes it on to
+// *report (when not NULL), which the host reads.
 __global__ __launch_bounds__(kUnpackLanes) void unpack_kernel(const UnpackRec* __restrict__ recs,
                                                             const uint32_t* __restrict__ start,
                                                             const uint32_t* __restrict__ hint,
                                                             const uint8_t* __restrict__ img,
-                                                            uint64_t img_bytes, uint32_t block0) {
+                                                            uint64_t img_bytes, uint32_t block0,
+                                                            uint32_t blocks,
+                                                            const uint32_t* __restrict__ bad,
+                                                            uint32_t* __restrict__ report) {
   const uint32_t blk = block0 + blockIdx.x;
+  const uint32_t failed = *bad;
+  if (report && blk == 0 && threadIdx.x == 0) *report = failed;
+  if (failed != kNoFailure || blk >= blocks) return;
   const uint32_t r = find_rec(start, hint, blk);
   const UnpackRec s = recs[r];
   const uint64_t e_begin = (uint64_t)(blk - start[r]) * unpack_seg(s.ftype);
@@ -593,23 +610,23 @@ DynHdr make_dyn(uint64_t gs, uint64_t as, int32_t n, const ark_opt_state* amp,
   return d;
 }
 
-// Queues the header kernel and the data kernels of a pack whose tables sit
-// at dtab (device, laid out as PackTables::host).
+// Queues the pack whose tables sit at dtab (device, laid out as
+// PackTables::host), the headers with its first launch.
 int launch_pack(const uint8_t* dtab, const PackTables& t, const DynHdr& dyn, uint8_t* img,
                 hipStream_t stream) {
-  const uint32_t nh = t.npieces + 1;
-  hipLaunchKernelGGL(header_kernel, dim3((nh + kThreads - 1) / kThreads), dim3(kThreads), 0,
-                     stream, (const HdrPiece*)dtab, t.npieces, dyn, img);
-  ARK_HIP(hipGetLastError());
   // a launch's work-items stay below 2^32: images past 64 GiB take several
-  const uint64_t per_launch = launch_blocks(kPackMaxBlocks);
-  for (uint64_t b0 = 0; b0 < t.blocks; b0 += per_launch) {
+  const uint32_t hb = (t.npieces + 1 + kPackLanes - 1) / kPackLanes;
+  const uint64_t per_launch = launch_blocks(kPackMaxBlocks - hb);
+  uint64_t b0 = 0;
+  do {
     const uint64_t nb = t.blocks - b0 < per_launch ? t.blocks - b0 : per_launch;
-    hipLaunchKernelGGL(pack_kernel, dim3((uint32_t)nb), dim3(kPackLanes), 0, stream,
-                       (const PackRec*)(dtab + t.recs_off), (const uint32_t*)(dtab + t.start_off),
-                       (const uint32_t*)(dtab + t.hint_off), img, (uint32_t)b0);
+    hipLaunchKernelGGL(pack_kernel, dim3((uint32_t)nb + (b0 ? 0u : hb)), dim3(kPackLanes), 0,
+                       stream, (const PackRec*)(dtab + t.recs_off),
+                       (const uint32_t*)(dtab + t.start_off), (const uint32_t*)(dtab + t.hint_off),
+                       img, (uint32_t)b0, (uint32_t)nb, (const HdrPiece*)dtab, t.npieces, dyn);
     ARK_HIP(hipGetLastError());
-  }
+    b0 += nb;
+  } while (b0 < t.blocks);
   return ARK_OPT_OK;
 }
 
@@ -654,11 +671,12 @@ int pack_image(const ark_ckpt_record* r, int32_t n, uint64_t gs, uint64_t as,
   return ARK_OPT_OK;
 }
 
-// Unpack descriptors of every record, grouped by file type, launched and
-// waited for.
+// Unpack descriptors of every record, launched and waited for.  checks: NULL,
+// or the headers to check first, on the device: when one fails nothing is
+// written and *failed is its index (kNoFailure otherwise).
 int unpack_image(const uint8_t* img, uint64_t img_bytes, const ark_ckpt_record* r, int32_t n,
-                 const std::vector<uint64_t>& data_off, const std::vector<uint32_t>& ftype,
-                 hipStream_t stream) {
+                 const std::vector<uint64_t>& data_off, const uint32_t* ftype,
+                 const std::vector<CheckDesc>* checks, uint32_t* failed, hipStream_t stream) {
   std::vector<UnpackRec> recs((size_t)n);
   std::vector<uint32_t> start((size_t)n + 1);
   uint64_t blocks = 0;
@@ -676,7 +694,7 @@ int unpack_image(const uint8_t* img, uint64_t img_bytes, const ark_ckpt_record* 
     if (blocks > 0x7FFFFFFFu) return fail(ARK_OPT_EINVAL, "checkpoint too large");
   }
   start[n] = (uint32_t)blocks;
-  if (blocks == 0) return ARK_OPT_OK;
+  if (blocks == 0 && !checks) return ARK_OPT_OK;
   {
     // a record's buffer may be an optimizer's gradient
     std::vector<const void*> dst((size_t)n);
@@ -687,13 +705,19 @@ int unpack_image(const uint8_t* img, uint64_t img_bytes, const ark_ckpt_record* 
     }
     ark::opt_units_invalidate(dst.data(), bytes.data(), (size_t)n);
   }
-  const std::vector<uint32_t> hint = make_hints(start, (uint32_t)n, blocks);
-  const size_t rb = recs.size() * sizeof(UnpackRec), stb = start.size() * sizeof(uint32_t);
-  const size_t hb = hint.size() * sizeof(uint32_t);
-  std::vector<uint8_t> host(rb + stb + hb);
-  memcpy(host.data(), recs.data(), rb);
-  memcpy(host.data() + rb, start.data(), stb);
-  memcpy(host.data() + rb + stb, hint.data(), hb);
+  // one upload: the tensors, the headers to check, the block starts and hints,
+  // and the failure index
+  const std::vector<uint32_t> hint =
+      blocks ? make_hints(start, (uint32_t)n, blocks) : std::vector<uint32_t>();
+  const size_t rb = recs.size() * sizeof(UnpackRec);
+  const size_t cb = checks ? checks->size() * sizeof(CheckDesc) : 0;
+  const size_t stb = start.size() * sizeof(uint32_t), hb = hint.size() * sizeof(uint32_t);
+  std::vector<uint8_t> host(rb + cb + stb + hb + sizeof(uint32_t));
+  if (rb) memcpy(host.data(), recs.data(), rb);
+  if (cb) memcpy(host.data() + rb, checks->data(), cb);
+  memcpy(host.data() + rb + cb, start.data(), stb);
+  if (hb) memcpy(host.data() + rb + cb + stb, hint.data(), hb);
+  memcpy(host.data() + rb + cb + stb + hb, &kNoFailure, sizeof(uint32_t));
   StreamBuf d;
   hipError_t e = d.alloc(host.size(), stream);
   if (e != hipSuccess) {
@@ -702,17 +726,34 @@ int unpack_image(const uint8_t* img, uint64_t img_bytes, const ark_ckpt_record* 
                 host.size());
   }
   StreamSync sync{stream};
-  ARK_HIP(hipMemcpyAsync(d.p, host.data(), host.size(), hipMemcpyHostToDevice, stream));
-  // a launch's work-items stay below 2^32: checkpoints past 128 GiB take several
-  const uint64_t per_launch = launch_blocks(kUnpackMaxBlocks);
-  for (uint64_t b0 = 0; b0 < blocks; b0 += per_launch) {
-    const uint64_t nb = blocks - b0 < per_launch ? blocks - b0 : per_launch;
-    hipLaunchKernelGGL(unpack_kernel, dim3((uint32_t)nb), dim3(kUnpackLanes), 0, stream,
-                       (const UnpackRec*)d.p, (const uint32_t*)((char*)d.p + rb),
-                       (const uint32_t*)((char*)d.p + rb + stb), img, img_bytes, (uint32_t)b0);
+  char* dev = (char*)d.p;
+  uint32_t* dbad = (uint32_t*)(dev + rb + cb + stb + hb);
+  ARK_HIP(hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, stream));
+  uint32_t* report = nullptr;
+  if (checks) {
+    report = (uint32_t*)d.host();
+    hipLaunchKernelGGL(check_kernel, dim3((uint32_t)(n + 1 + kThreads - 1) / kThreads),
+                       dim3(kThreads), 0, stream, (const CheckDesc*)(dev + rb), (uint32_t)n, img,
+                       dbad);
     ARK_HIP(hipGetLastError());
   }
+  // a launch's work-items stay below 2^32: checkpoints past 128 GiB take several
+  const uint64_t per_launch = launch_blocks(kUnpackMaxBlocks);
+  uint64_t b0 = 0;
+  do {
+    const uint64_t nb = blocks - b0 < per_launch ? blocks - b0 : per_launch;
+    hipLaunchKernelGGL(unpack_kernel, dim3(nb ? (uint32_t)nb : 1u), dim3(kUnpackLanes), 0, stream,
+                       (const UnpackRec*)dev, (const uint32_t*)(dev + rb + cb),
+                       (const uint32_t*)(dev + rb + cb + stb), img, img_bytes, (uint32_t)b0,
+                       (uint32_t)blocks, dbad, report);
+    ARK_HIP(hipGetLastError());
+    b0 += nb;
+  } while (b0 < blocks);
+  uint32_t x = kNoFailure;
+  if (checks && !report)
+    ARK_HIP(hipMemcpyAsync(&x, dbad, sizeof(x), hipMemcpyDeviceToHost, stream));
   ARK_HIP(hipStreamSynchronize(stream));
+  if (checks) *failed = report ? *report : x;
   return ARK_OPT_OK;
 }
 
@@ -1037,38 +1078,19 @@ int ark_ckpt_v4_unpack(const void* image, uint64_t image_bytes, const ark_ckpt_r
   if ((uintptr_t)image & 15u) return fail(ARK_OPT_EINVAL, "image not 16-byte aligned");
   if ((rc = ark::check_buffer(image, image_bytes, "image", 0))) return rc;
   hipStream_t s = (hipStream_t)stream;
-  // header check on the device
+  // the headers are checked on the device, before anything is written
   std::vector<CheckDesc> cd((size_t)n);
   for (int32_t i = 0; i < n; ++i) cd[i] = CheckDesc{L.hdr[i], records[i].n, file_types[i], 0};
-  // one upload: the header descriptors, then the failure index (all ones:
-  // no failure)
-  const size_t cb = cd.size() * sizeof(CheckDesc);
-  std::vector<uint8_t> host(cb + 16, 0xFF);
-  if (cb) memcpy(host.data(), cd.data(), cb);
-  StreamBuf d;
-  hipError_t e = d.alloc(host.size(), s);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    return fail(ARK_OPT_ENOMEM, "hipMallocAsync(%zu) for checkpoint descriptors failed",
-                host.size());
-  }
-  StreamSync sync{s};
-  uint32_t* dbad = (uint32_t*)((char*)d.p + cb);
-  ARK_HIP(hipMemcpyAsync(d.p, host.data(), host.size(), hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(check_kernel, dim3((uint32_t)(n + 1 + kThreads - 1) / kThreads),
-                     dim3(kThreads), 0, s, (const CheckDesc*)d.p, (uint32_t)n,
-                     (const uint8_t*)image, dbad);
-  ARK_HIP(hipGetLastError());
-  uint32_t bad = 0;
-  ARK_HIP(hipMemcpyAsync(&bad, dbad, 4, hipMemcpyDeviceToHost, s));
-  ARK_HIP(hipStreamSynchronize(s));
+  uint32_t bad = kNoFailure;
+  if ((rc = unpack_image((const uint8_t*)image, image_bytes, records, n, L.data, file_types, &cd,
+                         &bad, s)))
+    return rc;
   if (bad == (uint32_t)n)
     return fail(ARK_OPT_EIO, "image: V4 file header missing or n_tensors != %d", n);
-  if (bad != 0xFFFFFFFFu)
+  if (bad != kNoFailure)
     return fail(ARK_OPT_EIO, "image: tensor %u header does not match the record (n=%llu)", bad,
                 (unsigned long long)records[bad].n);
-  std::vector<uint32_t> ft(file_types, file_types + n);
-  return unpack_image((const uint8_t*)image, image_bytes, records, n, L.data, ft, s);
+  return ARK_OPT_OK;
 }
 
 int ark_ckpt_save_v4(const char* path, uint64_t global_step, uint64_t adam_step,
@@ -1264,7 +1286,8 @@ int ark_ckpt_load(const char* path, const ark_ckpt_record* records, int32_t n,
     ARK_HIP(hipMemcpyAsync((char*)img.p + off, pin[k & 1].p, len, hipMemcpyHostToDevice, s));
     ARK_HIP(hipEventRecord(ev[k & 1], s));
   }
-  if ((rc = unpack_image((const uint8_t*)img.p, total, records, n, P.data, P.type, s)))
+  if ((rc = unpack_image((const uint8_t*)img.p, total, records, n, P.data,
+                         P.type.data(), nullptr, nullptr, s)))
     return rc;
   if (info) *info = P.info;
   if (amp && P.info.has_amp) *amp = P.amp;
