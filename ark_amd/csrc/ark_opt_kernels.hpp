@@ -100,7 +100,7 @@ __host__ __device__ inline float lr_eff_of(float lr, float beta1, float beta2,
 }
 
 // Segments per norm block: 2 for fp16 gradients, 8 for fp32 (4 or 8 past
-// kMaxParts partials); halved while fewer than 512 blocks would cover the
+// kMaxParts partials); halved while fewer than 2048 blocks would cover the
 // table.
 int sumsq_spb(uint64_t nseg, uint32_t grad_dtype);
 // Group sums the norm pass's finalizer holds, and the most partials it takes
