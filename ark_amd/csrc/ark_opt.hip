@@ -61,7 +61,7 @@ struct ark_opt_handle {
   uint32_t norm_blocks = 0;
   uint32_t nt_from = 0;  // norm blocks from here up stream past the cache
   uint32_t sumsq_lds = 0;  // dynamic LDS per norm block (residency cap)
-  uint32_t adamw_lds = 0;  // dynamic LDS per AdamW block (residency cap)
+  uint32_t adamw_lds[2] = {0, 0};  // dynamic LDS per AdamW block (residency cap): [1] from units
   // one device allocation carved into the pieces below
   void* dev_mem = nullptr;
   SegDesc* d_segs = nullptr;
@@ -244,10 +244,11 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
     const int v = atoi(env);
     if (v == 0 || (v >= 2 && v <= 8)) sumsq_per_cu = v;
   }
-  int adamw_per_cu = ark::kAdamwWavesPerCu;
+  int adamw_per_cu[2] = {ark::adamw_waves(nseg, hp->grad_dtype, false),
+                         ark::adamw_waves(nseg, hp->grad_dtype, true)};
   if (const char* env = getenv("ARK_OPT_ADAMW_BLOCKS_PER_CU")) {
     const int v = atoi(env);
-    if (v == 0 || (v >= 4 && v <= 32)) adamw_per_cu = v;
+    if (v == 0 || (v >= 4 && v <= 32)) adamw_per_cu[0] = adamw_per_cu[1] = v;
   }
 
   // The reference steps distinct per-tensor fields (optimizer.rs:171,
@@ -296,7 +297,8 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
   h->norm_blocks = (uint32_t)parts;
   h->nt_from = ark::sumsq_nt_from(spb, gsz);
   h->sumsq_lds = ark::sumsq_lds_for(hp->grad_dtype, spb, sumsq_per_cu);
-  h->adamw_lds = ark::adamw_lds_for(hp->grad_dtype, adamw_per_cu);
+  for (int k = 0; k < 2; ++k)
+    h->adamw_lds[k] = ark::adamw_lds_for(hp->grad_dtype, adamw_per_cu[k]);
 
   // One allocation: segments | partial sums | state | scalars | info | units
   size_t off = 0;
@@ -396,7 +398,8 @@ int step_impl(ark_opt_handle* h, float lr, const float* lr_dev, ark_opt_step_inf
   fin.scal = h->d_scal;
   fin.host_info = info ? h->h_info : nullptr;
   fin.hp = h->hp;
-  if (take_fresh_units(h)) {
+  const bool from_units = take_fresh_units(h);
+  if (from_units) {
     // the gradients' producers already formed the tree's first level
     ARK_HIP(ark::launch_units_reduce(h->spb, h->d_units, h->d_segs, h->nseg, fin, h->stream));
   } else {
@@ -409,7 +412,8 @@ int step_impl(ark_opt_handle* h, float lr, const float* lr_dev, ark_opt_step_inf
   }
   if (h->nseg) {
     ARK_HIP(ark::launch_adamw(h->hp.grad_dtype, h->d_segs, h->nseg, h->d_scal,
-                              h->hp.beta1, h->hp.beta2, h->hp.eps, h->adamw_lds, h->stream));
+                              h->hp.beta1, h->hp.beta2, h->hp.eps, h->adamw_lds[from_units],
+                              h->stream));
   }
   if (ev) {
     ARK_HIP(hipEventRecord(ev[3], h->stream));

@@ -155,11 +155,33 @@ constexpr int kSumsqBlocksPerCuF16 = 7;
 // The dynamic LDS that holds the norm kernel for (grad_dtype, spb) at
 // `blocks` per CU (resident_lds_bytes; 0 = no cap).
 uint32_t sumsq_lds_for(uint32_t grad_dtype, int spb, int blocks);
-// Resident AdamW waves per CU.  32 (every wave slot) over-issue the pass's
-// seven streams: on MI355X the EKO-237M step takes 857 us unbounded, 844 at 24
-// per CU, 833-855 at 20 and 16 (the spread is where the buffers lie), 866 at 12;
-// the 1.3B set's 4732 at 20, 4522-4588 at 16.
-constexpr int kAdamwWavesPerCu = 16;
+// Resident AdamW waves per CU for a table of nseg segments, held by a
+// dynamic-LDS reservation: more waves hide the latency of what the norm pass
+// left in the Infinity Cache, but over-issue the seven streams that come from
+// HBM, so the fewer the larger the uncached share; a step from units finds
+// nothing cached.  Measured on MI355X, step in us with 12 / 16 / 20 / 24 waves
+// (two tables in turn):
+//   fp16 gradients   45M parameters   171.6   163.8   163.4   163.3
+//                    131M             475.4   456.1   454.1   456.1
+//                    237M             858.3   831.2   831.9   835.8  (alone 831.6 with 16, 837.4 with 20)
+//                    270M             997.2   968.2   971.9   979.3
+//                    1.3B            4677    4644    4714    4715
+//   fp32 gradients   20M               97.7    95.0    93.0    92.7
+//                    131M             559.4   552.4   549.9   550.3
+//                    270M            1169.0  1163.7  1158.4  1168.6
+//                    310M            1329.5  1321.5  1324.8  1331.5
+//                    404M            1736.2  1751.8  1749.1  1754.9
+//                    640M            2747    2770    2790    2802
+//   from units       10M (with the     88.2    88.6    88.5    88.5
+//                    237M hand-off)  1315.7  1320.9  1322.6  1329.8
+// A skipped step also dispatches faster with a smaller reservation (237M: 186,
+// 166, 159, 147 us).
+inline int adamw_waves(uint64_t nseg, uint32_t grad_dtype, bool from_units) {
+  if (from_units) return 12;
+  if (nseg <= (1u << 14)) return 24;  // 67M parameters
+  if (grad_dtype == ARK_OPT_GRAD_F16) return nseg <= (1u << 15) ? 20 : 16;  // 134M
+  return nseg <= (1u << 16) ? 20 : nseg <= 3u << 15 ? 16 : 12;              // 268M, 403M
+}
 // The dynamic LDS that holds the AdamW kernel for grad_dtype at `waves` per
 // CU, rounded up to whole blocks (resident_lds_bytes; 0 = no cap).
 uint32_t adamw_lds_for(uint32_t grad_dtype, int waves);
