@@ -404,8 +404,8 @@ __device__ __forceinline__ void fast_batch(const SegDesc (&dsc)[kRed], int tid, 
 }
 
 // Block 0 is the finalizer.  The others cover segments [b*SPB, b*SPB + SPB)
-// (SPB <= 8) each, b counted from the last, and publish the pairwise tree of their 2*SPB half-segment sums: an aligned subtree of the
-// global tree.  A block that saw an inf or NaN gradient writes NaN, so the
+// (SPB <= 8) each, b counted from the last, and publish the pairwise tree of
+// their 2*SPB half-segment sums: an aligned subtree of the global tree.  A block that saw an inf or NaN gradient writes NaN, so the
 // global sum is NaN exactly when some gradient is non-finite (training.rs:291).
 // Blocks from nt_from up read with non-temporal loads: they run first, and
 // what they read would leave the Infinity Cache before the AdamW pass gets
@@ -852,7 +852,7 @@ __global__ __launch_bounds__(kBlock) void clip_norm_kernel(const float* __restri
   }
 }
 
-// fold_kernel over nparts partials read as zero past the last one.
+// One level of the tree: aligned groups of kFoldGroup partials, zero past the last.
 __global__ __launch_bounds__(kFoldGroup) void clip_fold_kernel(const double* __restrict__ in,
                                                                uint32_t nparts,
                                                                double* __restrict__ out) {
