@@ -213,10 +213,22 @@ __device__ __forceinline__ void publish(double* slot, double x) {
   __hip_atomic_store((ARK_GLOBAL uint64_t*)slot, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Pairwise tree over 64 * R values in index order, lane l holding values l,
+// 64 + l, ... (so that every access to them is one contiguous stretch):
+// transpose_reduce turns the R trees over the lanes into one value per lane,
+// whose index has its bits in the lane's reversed.
+template <int R>
+__device__ __forceinline__ double group_tree(double (&q)[R], uint32_t lane) {
+  int idx = 0;
+  transpose_reduce<R, 0>(q, (int)lane, idx);
+  double x = butterfly_from<log2i(R)>(q[0]);
+#pragma unroll
+  for (int st = log2i(R) - 1; st >= 0; --st) x = x + __shfl_xor(x, 1 << st);
+  return x;
+}
+
 // Pairwise tree over the 64 * R partials of one group (0 past nparts) when all
-// have been published.  Lane l takes partials l, 64 + l, ...: every access is
-// one contiguous stretch, and transpose_reduce turns the R trees over the lanes
-// into one value per lane, whose index has its bits in the lane's reversed.
+// have been published.
 template <int R>
 __device__ __forceinline__ double take_group(double* __restrict__ part, uint32_t nparts,
                                              uint32_t group, uint32_t lane) {
@@ -243,12 +255,7 @@ __device__ __forceinline__ double take_group(double* __restrict__ part, uint32_t
       __hip_atomic_store(p + i0 + r * 64u, kUnset, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     q[r] = __builtin_bit_cast(double, v[r]);
   }
-  int idx = 0;
-  transpose_reduce<R, 0>(q, (int)lane, idx);
-  double x = butterfly_from<log2i(R)>(q[0]);
-#pragma unroll
-  for (int st = log2i(R) - 1; st >= 0; --st) x = x + __shfl_xor(x, 1 << st);
-  return x;
+  return group_tree<R>(q, lane);
 }
 
 // The root of the tree over the nparts partials, in wave 0.  The norm blocks
@@ -868,25 +875,21 @@ __global__ __launch_bounds__(kFoldGroup) void clip_fold_kernel(const double* __r
 // threshold (fcmp + b.le: an unordered compare does not clip), coefficient
 // threshold / norm; then g[i] = g[i] * coef (fmul, opti.s:409-420) over its share,
 // grid-stride over 4-element groups, or nothing.  Block 0 reports the norm.  The
-// leaves (24 KB for 24.6M values) come from the L2s in about the time a launch
-// of its own for the decision took to start (3.9 us and a gap on MI355X).
+// leaves (24 KB for 24.6M values) come from the L2s, a wave's 64 in one stretch
+// per load.  Measured on MI355X at 24.6M values, a call that does not clip 5.4 us
+// and one that does 35.6 (11.5 and 38.3 with L consecutive leaves per lane; a
+// launch of its own for the decision took 3.9 us and a gap).
 template <int L>
 __global__ __launch_bounds__(kBlock) void clip_scale_kernel(
     float* __restrict__ g, uint64_t n, uint32_t vec, const double* __restrict__ leaves,
     uint32_t nparts, float threshold, float* __restrict__ norm_out) {
   __shared__ double wsum[kBlock / 64];
   const uint32_t tid = threadIdx.x;
+  const uint32_t lane = tid & 63u, i0 = (tid >> 6) * 64u * L + lane;
   double q[L];
 #pragma unroll
-  for (int j = 0; j < L; ++j) {
-    const uint32_t i = tid * L + j;
-    q[j] = i < nparts ? leaves[i] : 0.0;
-  }
-#pragma unroll
-  for (int w = L / 2; w >= 1; w /= 2)
-#pragma unroll
-    for (int j = 0; j < w; ++j) q[j] = q[2 * j] + q[2 * j + 1];
-  const double x = butterfly_from<0>(q[0]);
+  for (int j = 0; j < L; ++j) q[j] = i0 + j * 64u < nparts ? leaves[i0 + j * 64u] : 0.0;
+  const double x = group_tree<L>(q, lane);
   if ((tid & 63u) == 0u) wsum[tid >> 6] = x;
   __syncthreads();
   const float norm = sqrtf((float)((wsum[0] + wsum[1]) + (wsum[2] + wsum[3])));
