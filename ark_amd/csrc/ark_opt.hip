@@ -49,6 +49,13 @@ int check_hparams(const ark_opt_hparams* hp) {
 
 constexpr int kTimingPool = 256;
 
+// ARK_OPT_FIN_POLLS=k: a test knob, so that a test can have the finalizer give
+// a step up; read at each step of a handle created while it was set.
+uint32_t fin_max_polls() {
+  const char* env = getenv("ARK_OPT_FIN_POLLS");
+  return env ? (uint32_t)strtoul(env, nullptr, 10) : ark::kFinMaxPolls;
+}
+
 }  // namespace
 
 struct ark_opt_handle {
@@ -59,13 +66,13 @@ struct ark_opt_handle {
   uint32_t nseg = 0;
   int spb = 2;
   uint32_t norm_blocks = 0;
+  bool fin_polls_knob = false;  // ARK_OPT_FIN_POLLS was set at create
   uint32_t nt_from = 0;  // norm blocks from here up stream past the cache
   uint32_t sumsq_lds = 0;  // dynamic LDS per norm block (residency cap)
   uint32_t adamw_lds[2] = {0, 0};  // dynamic LDS per AdamW block (residency cap): [1] from units
   // one device allocation carved into the pieces below
   void* dev_mem = nullptr;
   SegDesc* d_segs = nullptr;
-  double* d_part_sum = nullptr;  // one slot per norm block
   ark_opt_state* d_state = nullptr;
   StepScalars* d_scal = nullptr;
   ark_opt_step_info* h_info = nullptr;  // pinned, written by the step's kernels when asked for
@@ -295,22 +302,24 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
   h->nseg = (uint32_t)nseg;
   h->spb = spb;
   h->norm_blocks = (uint32_t)parts;
+  h->fin_polls_knob = getenv("ARK_OPT_FIN_POLLS") != nullptr;
   h->nt_from = ark::sumsq_nt_from(spb, gsz);
   h->sumsq_lds = ark::sumsq_lds_for(hp->grad_dtype, spb, sumsq_per_cu);
   for (int k = 0; k < 2; ++k)
     h->adamw_lds[k] = ark::adamw_lds_for(hp->grad_dtype, adamw_per_cu[k]);
 
-  // One allocation: segments | partial sums | state | scalars | info | units
+  // One allocation: scalars and norm slots | segments | state | units.  The
+  // AdamW pass counts its rows from the slots' on, its table pointer from as
+  // many descriptors before the first, which fall among the slots.
   size_t off = 0;
+  const size_t o_scal = off;
+  const size_t slot_bytes = sizeof(double) * (size_t)ark::norm_slots((uint32_t)parts);
+  off = align_up(off + ark::kSlotsOffset + slot_bytes, 256);
+  segs.resize(ark::padded_segs((uint32_t)nseg), SegDesc{});
   const size_t o_seg = off;
-  off = align_up(off + sizeof(SegDesc) * (size_t)(nseg ? nseg : 1), 256);
-  const size_t psum_bytes = sizeof(double) * (size_t)(parts ? parts : 1);
-  const size_t o_psum = off;
-  off = align_up(off + psum_bytes, 256);
+  off = align_up(off + sizeof(SegDesc) * segs.size(), 256);
   const size_t o_state = off;
   off = align_up(off + sizeof(ark_opt_state), 256);
-  const size_t o_scal = off;
-  off = align_up(off + sizeof(StepScalars), 256);
   const size_t o_units = off;
   if (hp->grad_dtype == ARK_OPT_GRAD_F32)
     off = align_up(off + sizeof(double) * (size_t)nseg * ark::kUnitsPerSeg, 256);
@@ -323,7 +332,6 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
   }
   char* base = (char*)h->dev_mem;
   h->d_segs = (SegDesc*)(base + o_seg);
-  h->d_part_sum = (double*)(base + o_psum);
   h->d_state = (ark_opt_state*)(base + o_state);
   h->d_scal = (StepScalars*)(base + o_scal);
   if (hp->grad_dtype == ARK_OPT_GRAD_F32 && nseg) h->d_units = (double*)(base + o_units);
@@ -344,10 +352,11 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
   }
   ark_opt_state st{};
   st.loss_scale = hp->loss_scale_init;  // training.rs:120
-  StepScalars sc{};
+  const StepScalars sc{};
   e = hipSuccess;
-  if (nseg) e = hipMemcpy(h->d_segs, segs.data(), sizeof(SegDesc) * nseg, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemset(h->d_part_sum, 0xFF, psum_bytes);  // every slot unset
+  if (nseg) e = hipMemcpy(h->d_segs, segs.data(), sizeof(SegDesc) * segs.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess && slot_bytes)
+    e = hipMemset(ark::slots_of(h->d_scal), 0xFF, slot_bytes);  // every slot unset
   if (e == hipSuccess) e = hipMemcpy(h->d_state, &st, sizeof(st), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(h->d_scal, &sc, sizeof(sc), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
@@ -370,6 +379,10 @@ int ark_opt_destroy(ark_opt_handle* h) {
 static int finish_info(ark_opt_handle* h, ark_opt_step_info* info) {
   ARK_HIP(hipStreamSynchronize(h->stream));
   *info = *h->h_info;
+  if (info->status == ARK_OPT_EHIP)
+    return fail(ARK_OPT_EHIP,
+                "the norm pass did not get every partial sum and nothing was updated (did "
+                "another step or graph replay of this handle run at the same time?)");
   return info->status;
 }
 
@@ -390,8 +403,9 @@ int step_impl(ark_opt_handle* h, float lr, const float* lr_dev, ark_opt_step_inf
     ARK_HIP(hipEventRecord(ev[0], h->stream));
   }
   ark::FinalizeArgs fin{};
-  fin.part = h->d_part_sum;
+  fin.part = ark::slots_of(h->d_scal);
   fin.nparts = h->norm_blocks;
+  fin.max_polls = h->fin_polls_knob ? fin_max_polls() : ark::kFinMaxPolls;
   fin.lr = lr;
   fin.lr_ptr = lr_dev;
   fin.state = h->d_state;
@@ -411,7 +425,7 @@ int step_impl(ark_opt_handle* h, float lr, const float* lr_dev, ark_opt_step_inf
     ARK_HIP(hipEventRecord(ev[2], h->stream));
   }
   if (h->nseg) {
-    ARK_HIP(ark::launch_adamw(h->hp.grad_dtype, h->d_segs, h->nseg, h->d_scal,
+    ARK_HIP(ark::launch_adamw(h->hp.grad_dtype, h->d_segs, h->nseg, h->norm_blocks, h->d_scal,
                               h->hp.beta1, h->hp.beta2, h->hp.eps, h->adamw_lds[from_units],
                               h->stream));
   }

@@ -197,8 +197,11 @@ constexpr int log2i(int v) { return v <= 1 ? 0 : 1 + log2i(v / 2); }
 // decisions.  It is one block and the only one that waits, for blocks that wait
 // for nothing, so the grid always drains.  A partial travels in its own slot, a
 // 64-bit agent-scope store and load (both pass the XCDs' L2s by) of a slot that
-// holds kUnset until then, so no fence orders anything; the finalizer puts
-// kUnset back for the next step.  What it costs is the time from the last
+// holds kUnset until then, so no fence orders anything; the first waves of the
+// step's AdamW pass put kUnset back, so every pass starts from clear slots.  The
+// wait is bounded (FinalizeArgs::max_polls): where two runs of one handle
+// overlap, one's AdamW pass may clear partials the other's finalizer waits for,
+// whose step then ends with nothing updated.  What it costs is the time from the last
 // partial to the scalars.  Measured on MI355X, norm pass to scalars, us (a norm
 // kernel, past 8192 partials a fold, and a one-block finalize before): one
 // 768 x 768 tensor 4.8 (3.2 + 3.3 and a launch between), one layer 7.8 (5.7 +
@@ -228,14 +231,15 @@ __device__ __forceinline__ double group_tree(double (&q)[R], uint32_t lane) {
 }
 
 // Pairwise tree over the 64 * R partials of one group (0 past nparts) when all
-// have been published.
+// have been published; kUnset's value when some have not been after *max_polls
+// more looks at them, and then *max_polls is 0: the wave waits no more.
 template <int R>
-__device__ __forceinline__ double take_group(double* __restrict__ part, uint32_t nparts,
-                                             uint32_t group, uint32_t lane) {
-  ARK_GLOBAL uint64_t* p = (ARK_GLOBAL uint64_t*)part;
+__device__ __forceinline__ double take_group(const double* __restrict__ part, uint32_t nparts,
+                                             uint32_t group, uint32_t lane, uint32_t* max_polls) {
+  const ARK_GLOBAL uint64_t* p = (const ARK_GLOBAL uint64_t*)part;
   const uint32_t i0 = group * 64u * R + lane;
   uint64_t v[R];
-  for (;;) {
+  for (uint32_t polls = *max_polls;; --polls) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       v[r] = 0ull;
@@ -246,31 +250,32 @@ __device__ __forceinline__ double take_group(double* __restrict__ part, uint32_t
 #pragma unroll
     for (int r = 0; r < R; ++r) ready = ready && v[r] != kUnset;
     if (__all(ready)) break;
+    if (polls == 0u) {
+      *max_polls = 0u;
+      return __builtin_bit_cast(double, kUnset);
+    }
     __builtin_amdgcn_s_sleep(1);
   }
   double q[R];
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    if (i0 + r * 64u < nparts)
-      __hip_atomic_store(p + i0 + r * 64u, kUnset, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    q[r] = __builtin_bit_cast(double, v[r]);
-  }
+  for (int r = 0; r < R; ++r) q[r] = __builtin_bit_cast(double, v[r]);
   return group_tree<R>(q, lane);
 }
 
-// The root of the tree over the nparts partials, in wave 0.  The norm blocks
-// run from the last to the first, and so do the groups here; sums holds
-// kFinGroups values in LDS.
+// The root of the tree over the nparts partials, in wave 0; *lost is set in it
+// when a wave's wait ended without its partials (the root is a NaN then).  The
+// norm blocks run from the last to the first, and so do the groups here; sums
+// holds kFinGroups values in LDS.
 template <int R>
-__device__ __forceinline__ double take_all(double* __restrict__ part, uint32_t nparts,
-                                           double* sums) {
+__device__ __forceinline__ double take_all(const double* __restrict__ part, uint32_t nparts,
+                                           uint32_t max_polls, double* sums, bool* lost) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t groups = (nparts + 64u * R - 1u) / (64u * R);
   for (uint32_t i = threadIdx.x; i < kFinGroups; i += kBlock)
     if (i >= groups) sums[i] = 0.0;
   for (uint32_t k = wave; k < groups; k += kBlock / 64) {
-    const double x = take_group<R>(part, nparts, groups - 1u - k, lane);
+    const double x = take_group<R>(part, nparts, groups - 1u - k, lane, &max_polls);
     if (lane == 0) sums[groups - 1u - k] = x;
   }
   __syncthreads();
@@ -283,7 +288,14 @@ __device__ __forceinline__ double take_all(double* __restrict__ part, uint32_t n
   for (int w = kPer / 2; w >= 1; w /= 2)
 #pragma unroll
     for (int j = 0; j < w; ++j) q[j] = q[2 * j] + q[2 * j + 1];
-  return butterfly_from<0>(q[0]);
+  const double root = butterfly_from<0>(q[0]);
+  if (__builtin_expect(__any(__builtin_isnan(root)), 0)) {
+    bool unset = false;
+    for (int j = 0; j < kPer; ++j)
+      unset = unset || __builtin_bit_cast(uint64_t, sums[lane * kPer + j]) == kUnset;
+    *lost = __any(unset);
+  }
+  return root;
 }
 
 __device__ inline uint32_t amp_skip(const ark_opt_hparams& hp, ark_opt_state& st) {
@@ -312,14 +324,15 @@ __device__ __forceinline__ void finalize_step(const FinalizeArgs& a, double* sum
   const float inv = 1.0f / st.loss_scale;  // training.rs:244
   const float lr_eff = lr_eff_of(lr, hp.beta1, hp.beta2, st.t + 1u);
   double sumsq;
+  bool lost = false;
   // a round of the waves takes all partials of a small table, and few rounds
   // those of a large one
   if (a.nparts <= kBlock)
-    sumsq = take_all<1>(a.part, a.nparts, sums);
+    sumsq = take_all<1>(a.part, a.nparts, a.max_polls, sums, &lost);
   else if (a.nparts <= 4u * kBlock)
-    sumsq = take_all<4>(a.part, a.nparts, sums);
+    sumsq = take_all<4>(a.part, a.nparts, a.max_polls, sums, &lost);
   else
-    sumsq = take_all<kMaxR>(a.part, a.nparts, sums);
+    sumsq = take_all<kMaxR>(a.part, a.nparts, a.max_polls, sums, &lost);
   if (threadIdx.x != 0) return;
 
   const bool any_bad = __builtin_isnan(sumsq);
@@ -333,7 +346,10 @@ __device__ __forceinline__ void finalize_step(const FinalizeArgs& a, double* sum
   out.clip_coef = 1.0f;
   out.status = ARK_OPT_OK;
   out.inv_scale = inv;
-  if (st.early_stop) {
+  if (lost) {  // nothing changes
+    out.status = ARK_OPT_EHIP;
+    sc.lr = 0.0f;
+  } else if (st.early_stop) {
     out.status = ARK_OPT_EARLY_STOP;
   } else if (!(fabsf(lr) <= 3.402823466e38f)) {  // a non-finite lr: nothing changes
     out.status = ARK_OPT_EINVAL;
@@ -369,7 +385,7 @@ __device__ __forceinline__ void finalize_step(const FinalizeArgs& a, double* sum
     }
   }
   out.state = st;
-  *a.state = st;
+  if (!lost) *a.state = st;
   *a.scal = sc;
   if (a.host_info) *a.host_info = out;
 }
@@ -698,23 +714,32 @@ __device__ __forceinline__ void adam_row(uint16_t* w, const GT* g, float* m, flo
 // adjacent rows 877 / 191, on rows 64 apart 845 / 191; four waves 32 rows apart
 // 838 / 175, 16 apart 847, 64 apart 843, 128 apart 854; eight waves 852 / 181;
 // two rows per wave 850 / 155-190, four 872 / 140-160.
+// The rows below `first` are the norm pass's slots (slot_rows).  They are the
+// first, and a branch the compiler leaves out of line, because a leaving wave
+// costs what its few scalar instructions do (skipped step's pass, us: 80.9 both
+// ways; 81.1 and the applied pass 1.5 longer with them last, 82-85 with other
+// forms of the branch).
 template <typename GT>
 __global__ __launch_bounds__(64 * kAdamWaves) void adamw_kernel(
     const SegDesc* __restrict__ segs, const StepScalars* __restrict__ scal,
-    float beta1, float beta2, float eps, uint32_t row0, uint32_t nrows) {
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t row = row0 + blockIdx.x / kAdamStride * kAdamGroup + wave * kAdamStride +
-                       blockIdx.x % kAdamStride;
-  if (row >= nrows) return;
+    float beta1, float beta2, float eps, uint32_t first, uint64_t* __restrict__ slots) {
+  // the wave's first lane is 64 * wave
+  const uint32_t row = blockIdx.x / kAdamStride * kAdamGroup + blockIdx.x % kAdamStride +
+                       __builtin_amdgcn_readfirstlane(threadIdx.x) / (64u / kAdamStride);
+  if (__builtin_expect(row < first, 0)) {
+    st_g<uint64_t>(slots + row * 64u + (threadIdx.x & 63u), kUnset);
+    return;
+  }
   SegDesc d = segs[row / kRowsPerSeg];
   StepScalars sc = *scal;
   // Every field used below is in registers before the first branch, so the
   // wave waits for one round trip of scalar loads rather than a chain of
   // them (left alone, the compiler loads the step scalars, branches, then
-  // loads the descriptor).
-  asm volatile("" : "+s"(d.w), "+s"(d.g), "+s"(d.m), "+s"(d.v), "+s"(d.n), "+s"(d.wd),
-               "+s"(d.flags), "+s"(sc.applied), "+s"(sc.inv), "+s"(sc.coef), "+s"(sc.lr),
-               "+s"(sc.lr_eff), "+s"(sc.c1), "+s"(sc.c2));
+  // loads the descriptor).  As inputs alone, so that no copies follow the wait;
+  // d.tensor keeps its register from being loaded twice, behind a wait.
+  asm volatile("" ::"s"(d.w), "s"(d.g), "s"(d.m), "s"(d.v), "s"(d.n), "s"(d.wd), "s"(d.flags),
+               "s"(d.tensor), "s"(sc.applied), "s"(sc.inv), "s"(sc.coef), "s"(sc.lr),
+               "s"(sc.lr_eff), "s"(sc.c1), "s"(sc.c2));
   if (!sc.applied) return;  // skipped step: training.rs:293-305
   const uint32_t r0 = (row % kRowsPerSeg) * kRow;
   if (r0 >= d.n) return;  // row past the end of a short segment
@@ -1034,22 +1059,25 @@ uint32_t adamw_lds_for(uint32_t grad_dtype, int waves) {
 }
 
 hipError_t launch_adamw(uint32_t grad_dtype, const SegDesc* segs, uint32_t nseg,
-                        const StepScalars* scal, float beta1, float beta2,
+                        uint32_t nparts, StepScalars* scal, float beta1, float beta2,
                         float eps, uint32_t lds_bytes, hipStream_t stream) {
   if ((uint64_t)nseg > kMaxSegments) return hipErrorInvalidValue;
-  const uint32_t nrows = nseg * kRowsPerSeg;
+  const uint32_t first = slot_rows(nparts), end = first + padded_segs(nseg) * kRowsPerSeg;
   const dim3 block(64 * kAdamWaves);
   // a launch's work-items stay below 2^32: the largest tables take two
   constexpr uint32_t kMaxRows = (1u << 26) - kAdamGroup;
-  for (uint32_t row0 = 0; row0 < nrows; row0 += kMaxRows) {
-    const uint32_t rows = nrows - row0 < kMaxRows ? nrows - row0 : kMaxRows;
-    const dim3 grid((rows + kAdamGroup - 1) / kAdamGroup * kAdamStride);
+  for (uint32_t row0 = 0; row0 < end; row0 += kMaxRows) {
+    const uint32_t rows = end - row0 < kMaxRows ? end - row0 : kMaxRows;
+    const dim3 grid(rows / kAdamGroup * kAdamStride);
+    // a row's descriptor, counted from the launch's first row
+    const SegDesc* d = segs + row0 / kRowsPerSeg - first / kRowsPerSeg;
+    const uint32_t f = row0 ? 0u : first;
     if (grad_dtype == ARK_OPT_GRAD_F16)
-      hipLaunchKernelGGL((adamw_kernel<uint16_t>), grid, block, lds_bytes, stream, segs, scal,
-                         beta1, beta2, eps, row0, nrows);
+      hipLaunchKernelGGL((adamw_kernel<uint16_t>), grid, block, lds_bytes, stream, d, scal, beta1,
+                         beta2, eps, f, (uint64_t*)slots_of(scal));
     else
-      hipLaunchKernelGGL((adamw_kernel<float>), grid, block, lds_bytes, stream, segs, scal, beta1,
-                         beta2, eps, row0, nrows);
+      hipLaunchKernelGGL((adamw_kernel<float>), grid, block, lds_bytes, stream, d, scal, beta1,
+                         beta2, eps, f, (uint64_t*)slots_of(scal));
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

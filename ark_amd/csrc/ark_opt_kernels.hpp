@@ -11,7 +11,9 @@
 //                       and writes the step scalars.
 //   2. adamw_kernel   : the fused streaming update (22 B/param): unscale, clip
 //                       coefficient, AdamW with decoupled weight decay, fp16
-//                       weight requantisation; exits at once on a skipped step.
+//                      coefficient, AdamW with decoupled weight decay, fp16
+//                      weight requantisation; exits at once on a skipped step.
+//                      Its first waves clear the slots the partials went through.
 //
 // Every tensor is cut into ARK_OPT_NORM_SEGMENT-element segments, listed in
 // table order, each with a 48-byte descriptor holding its four pointers
@@ -75,6 +77,12 @@ struct StepScalars {
   float c2;      // 1 - beta2
 };
 
+// The norm pass's slots, one per partial, lie behind the scalars in memory.
+constexpr size_t kSlotsOffset = 256;
+inline double* slots_of(StepScalars* scal) {
+  return reinterpret_cast<double*>(reinterpret_cast<char*>(scal) + kSlotsOffset);
+}
+
 // beta^t by binary exponentiation, then lr_eff = (sqrt(bc2) / bc1) * lr, one
 // IEEE binary32 operation per step as in opti.s:223-258.  Compiled for host
 // and device; both round every operation to nearest even.
@@ -108,11 +116,19 @@ int sumsq_spb(uint64_t nseg, uint32_t grad_dtype);
 constexpr uint32_t kFinGroups = 1024;
 constexpr uint32_t kMaxParts = kFinGroups * 64u * 8u;
 
-// What the finalizer needs (block 0 of the norm pass).  part: nparts slots,
-// every byte 0xFF before the first step; the pass leaves them so.
+// How often a finalizer wave looks for the partials of one group (1024 at
+// most) before it gives the step up: each look is a round trip past the L2s and
+// a sleep, 0.7 to 1 us together on MI355X, so the wait lasts over ten seconds.
+// The norm pass of 1.2B parameters takes at most 13 looks at a group; what the
+// bound leaves room for is other work on the GPU that holds the pass back.
+constexpr uint32_t kFinMaxPolls = 1u << 24;
+
+// What the finalizer needs (block 0 of the norm pass).  part: the slots, every
+// byte 0xFF before the first step; a step's AdamW pass leaves them so.
 struct FinalizeArgs {
   double* part;
   uint32_t nparts;
+  uint32_t max_polls;  // kFinMaxPolls
   float lr;
   const float* lr_ptr;  // NULL, or a device scalar this step's lr is read from
   ark_opt_state* state;
@@ -128,6 +144,18 @@ constexpr uint32_t kFoldGroup = 64u;
 // adamw: one wave per row, 16 rows per segment; rows and work-items must stay
 // below 2^32 work-items.
 constexpr uint64_t kMaxSegments = (1ull << 32) / (64ull * kRowsPerSeg) - 1;
+// An AdamW pass launches whole groups of rows: first one row for every 64 slots
+// of the norm pass, which it puts back to unset (kUnset), then the table's,
+// whose descriptors are padded with empty ones.
+inline uint32_t slot_rows(uint32_t nparts) {
+  return ((nparts + 63u) / 64u + kAdamGroup - 1u) / kAdamGroup * kAdamGroup;
+}
+inline uint32_t norm_slots(uint32_t nparts) { return slot_rows(nparts) * 64u; }
+static_assert(kAdamGroup % kRowsPerSeg == 0, "a group covers whole segments");
+inline uint32_t padded_segs(uint32_t nseg) {
+  constexpr uint32_t kSegs = kAdamGroup / kRowsPerSeg;
+  return (nseg + kSegs - 1u) / kSegs * kSegs;
+}
 static_assert((kMaxSegments + 7) / 8 <= kMaxParts, "8 segments per norm block cover every table");
 
 // ---------------------------------------------------------------------------
@@ -200,7 +228,7 @@ inline uint32_t sumsq_nt_from(int spb, uint64_t grad_bytes) {
 
 // lds_bytes: dynamic LDS per block, the residency cap (adamw_lds_for).
 hipError_t launch_adamw(uint32_t grad_dtype, const SegDesc* segs,
-                        uint32_t nseg, const StepScalars* scal, float beta1,
+                        uint32_t nseg, uint32_t nparts, StepScalars* scal, float beta1,
                         float beta2, float eps, uint32_t lds_bytes, hipStream_t stream);
 
 // One tensor given by value (fp32 gradients used as given, no unscale or

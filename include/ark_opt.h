@@ -112,7 +112,8 @@ typedef struct ark_opt_step_info {
   int32_t applied;    /* 1: AdamW ran; 0: skipped (non-finite or early stop) */
   int32_t nonfinite;  /* a gradient held inf or NaN                           */
   int32_t clipped;    /* norm > grad_clip && norm > 0 (optimizer.rs:148)      */
-  int32_t status;     /* ARK_OPT_OK or ARK_OPT_EARLY_STOP                     */
+  int32_t status;     /* ARK_OPT_OK, ARK_OPT_EARLY_STOP, or ARK_OPT_EHIP when
+                         the step was lost (ark_opt_step)                      */
   double grad_sumsq;  /* f64 sum of squares of the unscaled gradients (NaN
                          when a gradient is non-finite)                       */
   float grad_norm;    /* sqrtf((float)grad_sumsq): pre-clip norm              */
@@ -184,7 +185,13 @@ int ark_opt_destroy(ark_opt_handle *h);
  * gradients, or the units the hand-off's final calls wrote
  * (include/ark_grad.h) when they are fresh; a capture keeps the choice it
  * saw, so capture the step together with the final calls that feed it, or
- * with neither. */
+ * with neither.
+ * Steps of one handle, replays of captured ones among them, must be ordered
+ * with each other (one stream, or events between streams): they share the
+ * handle's partial sums and state.  A step that does not get its partial sums
+ * because another one ran at the same time is lost: after a bounded wait of
+ * some ten seconds it ends with nothing updated, info reports ARK_OPT_EHIP
+ * (returned by the call), and the handle is ready for the next step. */
 int ark_opt_step(ark_opt_handle *h, float lr, ark_opt_step_info *info);
 
 /* ark_opt_step with this step's learning rate read from the device scalar

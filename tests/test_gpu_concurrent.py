@@ -65,3 +65,61 @@ def test_two_handles_on_two_streams():
         assert c["w"] == c["m"] == c["v"] == 0, (i, c)
         opts[i].close()
     dq.close(), gp.close()
+
+
+@pytest.mark.parametrize("source", ["f16", "f32", "units"])
+def test_a_norm_pass_that_misses_partials_ends_and_the_next_step_is_whole(source, monkeypatch):
+    """The norm pass's finalizer gives a step up after a bounded number of
+    looks at the partials (a step of the same handle running at the same time
+    may have taken them).  Forced from the host by allowing no second look
+    while thousands of blocks are still reading: the step ends, reports the
+    error and changes nothing, with and without info; the same handle's next
+    steps are, bit for bit, those of a handle that lost none."""
+    import torch
+    from ark_amd import _abi, grad, synth
+    from ark_amd._lib import ArkOptError
+    from ark_amd.eko import TensorSpec
+    from ark_amd.optimizer import AdamConfig, AmpConfig, Optimizer
+    cfg = AdamConfig(lr=3e-4, beta1=0.9, beta2=0.95, eps=1e-8, weight_decay=0.1, grad_clip=1.0)
+    amp = AmpConfig(loss_scale_init=1024.0)
+    monkeypatch.setenv("ARK_OPT_SUMSQ_SPB", "1")  # 24,415 partials: 47 groups, a tail
+    specs = [TensorSpec("a", (100_000_123,), True, False)]
+    dt = _abi.GRAD_F16 if source == "f16" else _abi.GRAD_F32
+    sets = [synth.problem(specs, 77, 0.1, [1e-3], 1024.0, grad_dtype=dt) for _ in range(2)]
+    whole = Optimizer(cfg, sets[1], amp)
+    monkeypatch.setenv("ARK_OPT_FIN_POLLS", "0")
+    opt = Optimizer(cfg, sets[0], amp)
+    plans = []
+    if source == "units":
+        zero = torch.zeros(specs[0].n, device="cuda")
+        plans = [grad.GradPlan([(ps.g(0), zero)]) for ps in sets]
+
+    def step(which, info):
+        if plans:
+            plans[which].run(final_for=(opt, whole)[which])
+        return (opt, whole)[which].step_all(info=info)
+
+    def same():
+        return all(torch.equal(getattr(sets[0], k).view(torch.uint8), getattr(sets[1], k).view(torch.uint8))
+                   for k in ("w_arena", "g_arena", "m_arena", "v_arena"))
+
+    def state(o):
+        return bytes(o.get_state())
+
+    before = state(opt)
+    for _ in range(2):
+        with pytest.raises(ArkOptError, match="partial sum") as e:
+            step(0, True)
+        assert e.value.code == _abi.EHIP
+        step(0, False)
+        torch.cuda.synchronize()
+        assert state(opt) == before
+    assert same()
+    monkeypatch.delenv("ARK_OPT_FIN_POLLS")
+    for _ in range(2):
+        _, a = step(0, True)
+        _, b = step(1, True)
+        assert a.applied == 1 and bytes(a) == bytes(b)
+    assert same()
+    for o in (opt, whole, *plans):
+        o.close()
