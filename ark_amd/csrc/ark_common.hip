@@ -262,9 +262,17 @@ bool call_setup_locked(int dev) {
   return true;
 }
 
+// Whether the work of a slot's last holder has ended.
+bool slot_done(const CallSlot& s) {
+  if (!s.recorded || hipEventQuery(s.done) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 // Takes a slot for work on stream: one this stream used last if there is one
-// (nothing to wait for), else the longest given back.  Returns its index and
-// sets *dev and *p, or -1.
+// (in its order anyway), else the longest given back of those whose work has
+// ended, so that no stream waits for another's.  hipStreamPerThread names
+// another stream on each thread.  Returns its index and sets *dev and *p, or -1.
 int call_slot_take(hipStream_t stream, int* dev, void** p) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
@@ -278,15 +286,22 @@ int call_slot_take(hipStream_t stream, int* dev, void** p) {
     std::lock_guard<std::mutex> lock(g_call_mu);
     if (!call_setup_locked(*dev)) return -1;
     CallScratch& C = g_call[*dev];
+    uint32_t no = 0;  // slots not to be had
     for (int i = 0; i < kCallSlots; ++i) {
-      if (C.slot[i].held) continue;
-      if (C.slot[i].recorded && C.slot[i].last == stream) {
+      const CallSlot& s = C.slot[i];
+      if (s.held)
+        no |= 1u << i;
+      else if (k < 0 && s.recorded && s.last == stream && stream != hipStreamPerThread)
         k = i;
-        break;
-      }
-      if (k < 0 || C.slot[i].stamp < C.slot[k].stamp) k = i;
     }
-    if (k < 0) return -1;
+    while (k < 0) {
+      for (int i = 0; i < kCallSlots; ++i)
+        if (!(no >> i & 1u) && (k < 0 || C.slot[i].stamp < C.slot[k].stamp)) k = i;
+      if (k < 0) return -1;
+      if (slot_done(C.slot[k])) break;
+      no |= 1u << k;
+      k = -1;
+    }
     C.slot[k].held = true;
     *p = C.base + (size_t)k * kCallSlotBytes;
   }

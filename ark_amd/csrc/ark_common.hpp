@@ -120,7 +120,8 @@ int grad_scratch_prepare(int dev);
 // a slot is held by one call at a time, on any thread; the owner's end
 // records the slot's event behind the work it queued, and the next holder's
 // stream waits for that event, so calls on different streams never overlap in
-// a slot.  More, all slots held, or a capturing stream (whose graph must own
+// a slot.  A slot goes to the stream that used it last, or to any once its work
+// has ended.  More, no such slot, or a capturing stream (whose graph must own
 // its memory) take the stream-ordered pool, freed in stream order.
 // Measured on MI355X, a scatter of 64 tokens queued back to back: 33 us of
 // host time a call with hipMallocAsync (the pool orders each reuse behind the

@@ -57,8 +57,8 @@ int ark_grad_plan_destroy(ark_grad_plan *plan);
  * batch_seq < 2^24, d <= 65535 * 256.  Stream ordered; the scratch it needs
  * (8 B per token, past 12288 tokens 16 B and 1 KiB per 4096) is one of eight
  * 512 KiB slots the library keeps per GPU, ordered between streams and
- * threads by the library, or, past that and under graph capture, comes from the
- * stream-ordered pool. */
+ * threads by the library, or, past that, with other streams' work unfinished in
+ * all of them and under graph capture, comes from the stream-ordered pool. */
 int ark_grad_embed_scatter(float *embed_grad, uint32_t vocab, uint32_t d,
                            const uint32_t *tokens, const float *dx0, uint32_t batch_seq,
                            void *stream);

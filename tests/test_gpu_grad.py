@@ -4,6 +4,8 @@ fp32 accumulation of every gradient buffer, the LM-head and gamma_final
 adds, and the token scatter-add into the embedding gradient with the loop's
 summation order; then the produced fp32 gradients through ark_opt_step
 against the oracle's optimizer."""
+import time
+
 import numpy as np
 import pytest
 
@@ -196,6 +198,61 @@ def test_scatter_workspaces_on_many_streams(threads):
     torch.cuda.synchronize()
     for k, (gg, _, _, want, _) in enumerate(jobs):
         np.testing.assert_array_equal(_bits(gg).reshape(vocab, d), want.view(np.uint32), err_msg=str(k))
+
+
+def test_scatter_does_not_wait_for_another_streams_unfinished_call():
+    """One stream's scatter still to come, behind a long-running kernel, and
+    its workspace the longest given back once seven more streams have had
+    theirs: a ninth stream's scatter ends before it, and all are right."""
+    torch = _torch()
+    rng = np.random.default_rng(9)
+    vocab, d, n = 300, 64, 500
+    tokens = _zipf_tokens(rng, n, vocab)
+    dx0 = rng.standard_normal((n, d)).astype(np.float32)
+    g = rng.standard_normal((vocab, d)).astype(np.float32)
+    want = g.copy()
+    oracle.embed_scatter(want, tokens, dx0)
+    tt, xx = torch.from_numpy(tokens.view(np.int32)).cuda(), torch.from_numpy(dx0).cuda()
+    gs = [torch.from_numpy(g).cuda() for _ in range(9)]
+    t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    torch.cuda._sleep(1000)
+    t0.record()
+    torch.cuda._sleep(1_000_000)
+    t1.record()
+    torch.cuda.synchronize()
+    half_second = int(500 * 1_000_000 / t0.elapsed_time(t1))  # in _sleep's unit
+    streams = [torch.cuda.Stream() for _ in range(20)]
+    mark = torch.zeros(8, device="cuda")
+
+    def ends_within(stream, seconds):
+        e = torch.cuda.Event()
+        e.record(stream)
+        end = time.perf_counter() + seconds
+        while not e.query() and time.perf_counter() < end:
+            pass
+        return e.query()
+
+    with torch.cuda.stream(streams[0]):
+        torch.cuda._sleep(half_second)
+    for s, gg in zip(streams, gs[:8]):
+        with torch.cuda.stream(s):
+            grad.embed_scatter(gg, tt, xx)
+    # streams share a few hardware queues: one whose work overtakes the first's
+    for s in streams[8:]:
+        with torch.cuda.stream(s):
+            mark.add_(1.0)
+        if ends_within(s, 0.01):
+            break
+    else:
+        pytest.skip("no stream of these runs beside the first")
+    with torch.cuda.stream(s):
+        grad.embed_scatter(gs[8], tt, xx)
+    overtook = ends_within(s, 0.1)
+    pending = not streams[0].query()
+    torch.cuda.synchronize()
+    assert pending and overtook, (pending, overtook)
+    for gg in gs:
+        np.testing.assert_array_equal(_bits(gg).reshape(vocab, d), want.view(np.uint32))
 
 
 @pytest.mark.parametrize("d,x_off", [(256, 0), (260, 0), (65, 0), (256, 1)])
