@@ -69,7 +69,8 @@ struct ark_opt_handle {
   bool fin_polls_knob = false;  // ARK_OPT_FIN_POLLS was set at create
   uint32_t nt_from = 0;  // norm blocks from here up stream past the cache
   uint32_t sumsq_lds = 0;  // dynamic LDS per norm block (residency cap)
-  uint32_t adamw_lds[2] = {0, 0};  // dynamic LDS per AdamW block (residency cap): [1] from units
+  uint32_t adamw_lds = 0;        // dynamic LDS per AdamW block (residency cap)
+  uint32_t adamw_units_lds = 0;  // the same for a step from units
   // one device allocation carved into the pieces below
   void* dev_mem = nullptr;
   SegDesc* d_segs = nullptr;
@@ -251,11 +252,11 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
     const int v = atoi(env);
     if (v == 0 || (v >= 2 && v <= 8)) sumsq_per_cu = v;
   }
-  int adamw_per_cu[2] = {ark::adamw_waves(nseg, hp->grad_dtype, false),
-                         ark::adamw_waves(nseg, hp->grad_dtype, true)};
+  int adamw_per_cu = ark::adamw_waves(nseg, hp->grad_dtype, false);
+  int adamw_units_per_cu = ark::adamw_waves(nseg, hp->grad_dtype, true);
   if (const char* env = getenv("ARK_OPT_ADAMW_BLOCKS_PER_CU")) {
     const int v = atoi(env);
-    if (v == 0 || (v >= 4 && v <= 32)) adamw_per_cu[0] = adamw_per_cu[1] = v;
+    if (v == 0 || (v >= 4 && v <= 32)) adamw_per_cu = adamw_units_per_cu = v;
   }
 
   // The reference steps distinct per-tensor fields (optimizer.rs:171,
@@ -305,8 +306,10 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
   h->fin_polls_knob = getenv("ARK_OPT_FIN_POLLS") != nullptr;
   h->nt_from = ark::sumsq_nt_from(spb, gsz);
   h->sumsq_lds = ark::sumsq_lds_for(hp->grad_dtype, spb, sumsq_per_cu);
-  for (int k = 0; k < 2; ++k)
-    h->adamw_lds[k] = ark::adamw_lds_for(hp->grad_dtype, adamw_per_cu[k]);
+  h->adamw_lds = ark::adamw_lds_for(hp->grad_dtype, adamw_per_cu);
+  h->adamw_units_lds = adamw_units_per_cu == adamw_per_cu
+                           ? h->adamw_lds
+                           : ark::adamw_lds_for(hp->grad_dtype, adamw_units_per_cu);
 
   // One allocation: scalars and norm slots | segments | state | units.  The
   // AdamW pass counts its rows from the slots' on, its table pointer from as
@@ -426,8 +429,8 @@ int step_impl(ark_opt_handle* h, float lr, const float* lr_dev, ark_opt_step_inf
   }
   if (h->nseg) {
     ARK_HIP(ark::launch_adamw(h->hp.grad_dtype, h->d_segs, h->nseg, h->norm_blocks, h->d_scal,
-                              h->hp.beta1, h->hp.beta2, h->hp.eps, h->adamw_lds[from_units],
-                              h->stream));
+                              h->hp.beta1, h->hp.beta2, h->hp.eps,
+                              from_units ? h->adamw_units_lds : h->adamw_lds, h->stream));
   }
   if (ev) {
     ARK_HIP(hipEventRecord(ev[3], h->stream));

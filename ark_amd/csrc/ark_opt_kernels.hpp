@@ -187,28 +187,31 @@ uint32_t sumsq_lds_for(uint32_t grad_dtype, int spb, int blocks);
 // dynamic-LDS reservation: more waves hide the latency of what the norm pass
 // left in the Infinity Cache, but over-issue the seven streams that come from
 // HBM, so the fewer the larger the uncached share; a step from units finds
-// nothing cached.  Measured on MI355X, step in us with 12 / 16 / 20 / 24 waves
-// (two tables in turn):
-//   fp16 gradients   45M parameters   171.6   163.8   163.4   163.3
-//                    131M             475.4   456.1   454.1   456.1
-//                    237M             858.3   831.2   831.9   835.8  (alone 831.6 with 16, 837.4 with 20)
-//                    270M             997.2   968.2   971.9   979.3
-//                    1.3B            4677    4644    4714    4715
-//   fp32 gradients   20M               97.7    95.0    93.0    92.7
-//                    131M             559.4   552.4   549.9   550.3
-//                    270M            1169.0  1163.7  1158.4  1168.6
-//                    310M            1329.5  1321.5  1324.8  1331.5
-//                    404M            1736.2  1751.8  1749.1  1754.9
-//                    640M            2747    2770    2790    2802
-//   from units       10M (with the     88.2    88.6    88.5    88.5
-//                    237M hand-off)  1315.7  1320.9  1322.6  1329.8
-// A skipped step also dispatches faster with a smaller reservation (237M: 186,
-// 166, 159, 147 us).
+// nothing cached.  Measured on MI355X, step in us (two tables in turn, 15
+// rounds in a random order; the rounds' 10th and 90th percentiles lie within
+// 0.2 % of the median):
+//   waves                     12       16       20       24
+//   fp16 gradients     7M     33.86    32.93    33.69    33.05
+//                      20M    80.63    78.90    78.66    78.26
+//                      45M   164.9    160.8    161.4    162.1
+//                      90M   325.2    314.7    315.2    318.1
+//                      131M  469.3    457.1    457.3    461.9
+//                      237M  849.7    829.0    832.6    840.1
+//   fp32 gradients     8M     40.14    39.66    39.06    38.81
+//                      20M    90.57    88.02    87.34    87.43
+//                      45M   192.4    187.7    185.7    186.0
+//                      90M   379.9    375.1    373.4    375.4
+//                      131M  550.1    547.7    547.1    550.0
+//                      270M 1149.8   1151.5   1151.4   1158.7
+//                      404M 1718.5   1722.2   1722.6   1729.8
+//                      640M 2713.6   2740.5   2746.2   2762.2
+//   from units         10M    62.77    62.96    62.65    62.60
+//   (with the          45M   254.5    255.8    256.0    256.7
+//   accumulation)      237M 1280.9   1291.5   1300.4   1303.3
 inline int adamw_waves(uint64_t nseg, uint32_t grad_dtype, bool from_units) {
-  if (from_units) return 12;
-  if (nseg <= (1u << 14)) return 24;  // 67M parameters
-  if (grad_dtype == ARK_OPT_GRAD_F16) return nseg <= (1u << 15) ? 20 : 16;  // 134M
-  return nseg <= (1u << 16) ? 20 : nseg <= 3u << 15 ? 16 : 12;              // 268M, 403M
+  if (grad_dtype == ARK_OPT_GRAD_F16) return 16;
+  if (from_units || nseg > (1u << 15)) return 12;  // 134M parameters
+  return nseg <= (1u << 12) ? 24 : 20;             // 17M
 }
 // The dynamic LDS that holds the AdamW kernel for grad_dtype at `waves` per
 // CU, rounded up to whole blocks (resident_lds_bytes; 0 = no cap).
