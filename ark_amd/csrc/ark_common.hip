@@ -190,6 +190,24 @@ uint32_t resident_lds_bytes(const void* kernel, int threads, int blocks) {
   }
   const uint32_t lds = (uint32_t)lds_per_cu(dev);
   if (lds == 0) return 0;
+  // found once per device, kernel and shape (a search is ~5 us of a handle's
+  // creation)
+  struct Found {
+    int dev;
+    const void* kernel;
+    int threads, blocks;
+    uint32_t bytes;
+  };
+  static std::mutex mu;
+  static std::vector<Found> found;
+  std::lock_guard<std::mutex> lock(mu);
+  for (const Found& f : found)
+    if (f.dev == dev && f.kernel == kernel && f.threads == threads && f.blocks == blocks)
+      return f.bytes;
+  auto keep = [&](uint32_t bytes) {
+    found.push_back({dev, kernel, threads, blocks, bytes});
+    return bytes;
+  };
   // resident blocks with `dyn` bytes reserved (0 when it cannot launch)
   auto occ = [&](uint32_t dyn, int* n) {
     *n = 0;
@@ -201,7 +219,8 @@ uint32_t resident_lds_bytes(const void* kernel, int threads, int blocks) {
     return true;
   };
   int n0 = 0;
-  if (!occ(0, &n0) || n0 <= blocks) return 0;
+  if (!occ(0, &n0)) return 0;
+  if (n0 <= blocks) return keep(0);
   // smallest reservation in (0, lds] that leaves at most b blocks
   auto first_at_most = [&](int b) {
     uint32_t lo = 0, hi = lds;  // occupancy(lo) > b >= occupancy(hi)
@@ -217,7 +236,7 @@ uint32_t resident_lds_bytes(const void* kernel, int threads, int blocks) {
     return hi;
   };
   const uint32_t a = first_at_most(blocks), z = first_at_most(blocks - 1);
-  return a + (z - a) / 2;
+  return keep(a + (z - a) / 2);
 }
 
 namespace {
