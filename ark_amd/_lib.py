@@ -127,11 +127,13 @@ def check(rc):
 
 def current_stream(t=None):
     """torch's current HIP stream (of t's device when t is given), as the
-    void* the C ABI takes.  Asked for by device number: torch's Stream object
-    costs 3 us, as much as queueing a kernel."""
+    void* the C ABI takes.  Asked for by device number where this torch has the
+    call, which is not public: torch's Stream object costs 3 us, as much as
+    queueing a kernel."""
     import torch
     dev = t.device.index if t is not None else torch.cuda.current_device()
-    return C.c_void_p(torch._C._cuda_getCurrentRawStream(dev))
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return C.c_void_p(raw(dev) if raw else torch.cuda.current_stream(dev).cuda_stream)
 
 
 def exported_symbols():

@@ -63,3 +63,25 @@ def test_param_arena_layout_on_cpu():
         assert t.weight_decay == float(np.float32(0.1 if ps.specs[i].decay else 0.0))
     assert tab[8].flags == _abi.TENSOR_NO_UNSCALE and tab[7].flags == 0
     assert ps.n_params == 7_079_424
+
+
+@pytest.mark.parametrize("raw_call", [True, False])
+def test_current_stream_with_and_without_torchs_raw_call(raw_call, monkeypatch):
+    """The stream of the tensor's device, or of the current one, also from a
+    torch that lacks the call by device number."""
+    import types
+
+    import torch
+    from ark_amd._lib import current_stream
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(torch.cuda, "current_stream",
+                        lambda dev: types.SimpleNamespace(cuda_stream=100 + dev))
+    if raw_call:
+        monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda dev: 200 + dev,
+                            raising=False)
+    else:
+        monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    base = 200 if raw_call else 100
+    t = types.SimpleNamespace(device=torch.device("cuda", 3))
+    assert current_stream(t).value == base + 3
+    assert current_stream().value == base + 1
