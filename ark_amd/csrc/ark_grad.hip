@@ -776,6 +776,17 @@ static_assert(kLongRun <= (uint32_t)kWave, "a lane for each row of a short run")
 constexpr uint32_t kMaxTokens = (1u << 24) - 1u;  // the call's limit (include/ark_grad.h)
 constexpr uint64_t kMaxRunBlocks = ((1ull << 32) - 1) / (kRunWaves * kWave);
 
+// ARK_GRAD_LAUNCH_POSITIONS=k (k >= kLongRun, taken down to a multiple of it)
+// caps the sorted positions per run_kernel launch (a test knob: it splits even
+// small batches over many launches, which must give the same bits).
+uint64_t launch_positions(uint64_t most) {
+  if (const char* env = getenv("ARK_GRAD_LAUNCH_POSITIONS")) {
+    const uint64_t v = strtoull(env, nullptr, 10) / kLongRun * kLongRun;
+    if (v && v < most) return v;
+  }
+  return most;
+}
+
 using ark::overlaps;
 
 using ark::StreamBuf;
@@ -848,7 +859,7 @@ void invalidate_embed_units(const float* embed_grad, uint32_t vocab, uint32_t d)
 }
 
 // Queues the scatter on s with its workspace at ws (L.bytes bytes, 256-byte
-// aligned): the sort, the row copy and the run adds.
+// aligned): the sort and the run adds.
 int scatter_launch(float* embed_grad, uint32_t vocab, uint32_t d, const uint32_t* tokens,
                    const float* dx0, uint32_t n, char* ws, const ScatterLayout& L,
                    hipStream_t s) {
@@ -892,7 +903,8 @@ int scatter_launch(float* embed_grad, uint32_t vocab, uint32_t d, const uint32_t
       (d % 4u) == 0 && ((((uintptr_t)embed_grad | (uintptr_t)dx0) & 15u) == 0);
   const uint64_t ctiles = (d + kWave - 1) / kWave, tiles = (d + kTileCols - 1) / kTileCols;
   // a launch's work-items stay below 2^32: past that many positions, several
-  uint64_t per = kMaxRunBlocks / (ctiles + kLongRun * tiles / kRunWaves + 1u) * kLongRun;
+  uint64_t per = launch_positions(
+      kMaxRunBlocks / (ctiles + kLongRun * tiles / kRunWaves + 1u) * kLongRun);
   if (per > n) per = n;
   for (uint64_t p0 = 0; p0 < n; p0 += per) {
     const uint64_t p1 = p0 + per < n ? p0 + per : n;

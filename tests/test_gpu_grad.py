@@ -161,6 +161,60 @@ def test_scatter_run_lengths_at_the_path_boundaries(d):
     np.testing.assert_array_equal(_bits(gg).reshape(vocab, d), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("final", [False, True])
+@pytest.mark.parametrize("d", [256, 260])
+@pytest.mark.parametrize("positions", [32, 64, 96])
+def test_scatter_runs_across_launch_boundaries(positions, d, final, monkeypatch):
+    """The sorted positions past a launch's work-items go over several
+    launches, here 32, 64 or 96 each: runs of 1 to 200 rows that start just
+    before, on and just after a boundary and end there too, some across several
+    launches, each taken exactly once.  final: through the call that also
+    writes the norm's units, whose step matches one that reads the gradients."""
+    from ark_amd import _abi
+    from ark_amd.eko import TensorSpec
+    from ark_amd.optimizer import AdamConfig, AmpConfig, Optimizer, ParamSet
+    torch = _torch()
+    monkeypatch.setenv("ARK_GRAD_LAUNCH_POSITIONS", str(positions))
+    rng = np.random.default_rng(positions + d)
+    # in sorted order: each run fills up to 1 below, at, or 1 past a boundary
+    lengths, at = [], 0
+    for k, past in enumerate([-1, 2, 0, 1, -1, 1, 0, -1, 33, 31, 32, 1, 0, 200, -1, 64, 1, 95, -1] * 3):
+        if past > 2:
+            n = past
+        else:
+            n = (at // positions + 1 + k % 2) * positions + past - at
+        lengths.append(n)
+        at += n
+    vocab = len(lengths) + 7
+    ids = np.sort(rng.choice(vocab, len(lengths), replace=False))
+    tokens = np.concatenate([np.full(k, t, np.uint32) for k, t in zip(lengths, ids)])
+    tokens = tokens[rng.permutation(len(tokens))]
+    n = len(tokens)
+    dx0 = (rng.standard_normal((n, d)) * 10.0 ** rng.integers(-4, 4, (n, 1))).astype(np.float32)
+    g = rng.standard_normal((vocab, d)).astype(np.float32)
+    want = g.copy()
+    oracle.embed_scatter(want, tokens, dx0)
+    tt, xx = torch.from_numpy(tokens.view(np.int32)).cuda(), torch.from_numpy(dx0).cuda()
+    if not final:
+        gg = torch.from_numpy(g).cuda()
+        grad.embed_scatter(gg, tt, xx)
+        np.testing.assert_array_equal(_bits(gg).reshape(vocab, d), want.view(np.uint32))
+        return
+    infos = []
+    for fused in (True, False):
+        ps = ParamSet([TensorSpec("embed", (vocab, d), True, False)], 0.1, grad_dtype=_abi.GRAD_F32)
+        src = torch.from_numpy(g).cuda().view(-1)
+        opt = Optimizer(AdamConfig(), ps, AmpConfig(loss_scale_init=256.0))
+        plan = grad.GradPlan([(ps.g(0), src)])
+        plan.run(final_for=opt if fused else None)
+        gg = ps.g(0).view(vocab, d)
+        grad.embed_scatter(gg, tt, xx, final_for=opt if fused else None)
+        infos.append(bytes(opt.step_all(3e-4, info=True)[1]))
+        np.testing.assert_array_equal(_bits(gg).reshape(vocab, d), want.view(np.uint32))
+        opt.close(), plan.close()
+    assert infos[0] == infos[1]
+
+
 @pytest.mark.parametrize("threads", [1, 4])
 def test_scatter_workspaces_on_many_streams(threads):
     """Twelve streams, more than the library keeps workspaces for, with
