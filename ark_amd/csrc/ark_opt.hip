@@ -70,6 +70,7 @@ struct ark_opt_handle {
   uint32_t nt_from = 0;  // norm blocks from here up stream past the cache
   uint32_t sumsq_lds = 0;  // dynamic LDS per norm block (residency cap)
   uint32_t adamw_lds = 0;        // dynamic LDS per AdamW block (residency cap)
+  uint32_t adamw_max_rows = ark::kAdamMaxRows;  // per launch
   uint32_t adamw_units_lds = 0;  // the same for a step from units
   // one device allocation carved into the pieces below
   void* dev_mem = nullptr;
@@ -303,6 +304,12 @@ int ark_opt_create(const ark_opt_tensor* tensors, int32_t n_tensors,
   h->nseg = (uint32_t)nseg;
   h->spb = spb;
   h->norm_blocks = (uint32_t)parts;
+  // ARK_OPT_ADAMW_LAUNCH_ROWS=k caps the rows per AdamW launch (a test knob: it
+  // splits even small tables over many launches, which must give the same bits)
+  if (const char* env = getenv("ARK_OPT_ADAMW_LAUNCH_ROWS")) {
+    const unsigned long long v = strtoull(env, nullptr, 10) / ark::kAdamGroup * ark::kAdamGroup;
+    if (v && v < ark::kAdamMaxRows) h->adamw_max_rows = (uint32_t)v;
+  }
   h->fin_polls_knob = getenv("ARK_OPT_FIN_POLLS") != nullptr;
   h->nt_from = ark::sumsq_nt_from(spb, gsz);
   h->sumsq_lds = ark::sumsq_lds_for(hp->grad_dtype, spb, sumsq_per_cu);
@@ -430,7 +437,8 @@ int step_impl(ark_opt_handle* h, float lr, const float* lr_dev, ark_opt_step_inf
   if (h->nseg) {
     ARK_HIP(ark::launch_adamw(h->hp.grad_dtype, h->d_segs, h->nseg, h->norm_blocks, h->d_scal,
                               h->hp.beta1, h->hp.beta2, h->hp.eps,
-                              from_units ? h->adamw_units_lds : h->adamw_lds, h->stream));
+                              from_units ? h->adamw_units_lds : h->adamw_lds, h->adamw_max_rows,
+                              h->stream));
   }
   if (ev) {
     ARK_HIP(hipEventRecord(ev[3], h->stream));

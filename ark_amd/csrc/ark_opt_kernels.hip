@@ -1060,24 +1060,24 @@ uint32_t adamw_lds_for(uint32_t grad_dtype, int waves) {
 
 hipError_t launch_adamw(uint32_t grad_dtype, const SegDesc* segs, uint32_t nseg,
                         uint32_t nparts, StepScalars* scal, float beta1, float beta2,
-                        float eps, uint32_t lds_bytes, hipStream_t stream) {
-  if ((uint64_t)nseg > kMaxSegments) return hipErrorInvalidValue;
+                        float eps, uint32_t lds_bytes, uint32_t max_rows, hipStream_t stream) {
+  if ((uint64_t)nseg > kMaxSegments || !max_rows || max_rows % kAdamGroup)
+    return hipErrorInvalidValue;
   const uint32_t first = slot_rows(nparts), end = first + padded_segs(nseg) * kRowsPerSeg;
   const dim3 block(64 * kAdamWaves);
-  // a launch's work-items stay below 2^32: the largest tables take two
-  constexpr uint32_t kMaxRows = (1u << 26) - kAdamGroup;
-  for (uint32_t row0 = 0; row0 < end; row0 += kMaxRows) {
-    const uint32_t rows = end - row0 < kMaxRows ? end - row0 : kMaxRows;
+  for (uint32_t row0 = 0; row0 < end; row0 += max_rows) {
+    const uint32_t rows = end - row0 < max_rows ? end - row0 : max_rows;
     const dim3 grid(rows / kAdamGroup * kAdamStride);
     // a row's descriptor, counted from the launch's first row
     const SegDesc* d = segs + row0 / kRowsPerSeg - first / kRowsPerSeg;
-    const uint32_t f = row0 ? 0u : first;
+    const uint32_t f = first > row0 ? first - row0 : 0u;
+    uint64_t* slots = (uint64_t*)slots_of(scal) + (uint64_t)row0 * 64u;
     if (grad_dtype == ARK_OPT_GRAD_F16)
       hipLaunchKernelGGL((adamw_kernel<uint16_t>), grid, block, lds_bytes, stream, d, scal, beta1,
-                         beta2, eps, f, (uint64_t*)slots_of(scal));
+                         beta2, eps, f, slots);
     else
       hipLaunchKernelGGL((adamw_kernel<float>), grid, block, lds_bytes, stream, d, scal, beta1,
-                         beta2, eps, f, (uint64_t*)slots_of(scal));
+                         beta2, eps, f, slots);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

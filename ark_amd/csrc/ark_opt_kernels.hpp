@@ -151,6 +151,9 @@ inline uint32_t slot_rows(uint32_t nparts) {
   return ((nparts + 63u) / 64u + kAdamGroup - 1u) / kAdamGroup * kAdamGroup;
 }
 inline uint32_t norm_slots(uint32_t nparts) { return slot_rows(nparts) * 64u; }
+// Most rows of one launch, whose work-items stay below 2^32: the largest tables
+// take two.
+constexpr uint32_t kAdamMaxRows = (1u << 26) - kAdamGroup;
 static_assert(kAdamGroup % kRowsPerSeg == 0, "a group covers whole segments");
 inline uint32_t padded_segs(uint32_t nseg) {
   constexpr uint32_t kSegs = kAdamGroup / kRowsPerSeg;
@@ -230,9 +233,11 @@ inline uint32_t sumsq_nt_from(int spb, uint64_t grad_bytes) {
 }
 
 // lds_bytes: dynamic LDS per block, the residency cap (adamw_lds_for).
+// max_rows: rows per launch, a multiple of kAdamGroup.
 hipError_t launch_adamw(uint32_t grad_dtype, const SegDesc* segs,
                         uint32_t nseg, uint32_t nparts, StepScalars* scal, float beta1,
-                        float beta2, float eps, uint32_t lds_bytes, hipStream_t stream);
+                        float beta2, float eps, uint32_t lds_bytes, uint32_t max_rows,
+                        hipStream_t stream);
 
 // One tensor given by value (fp32 gradients used as given, no unscale or
 // clip) with host-computed scalars: the drop-in of one

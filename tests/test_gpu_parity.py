@@ -150,6 +150,27 @@ def test_partial_counts_around_the_finalizers_groups(parts, grad_dtype, monkeypa
     opt.close()
 
 
+@pytest.mark.parametrize("rows", ["128", "256", "1024"])
+@pytest.mark.parametrize("grad_dtype", [_abi.GRAD_F16, _abi.GRAD_F32])
+def test_adamw_over_many_launches(grad_dtype, rows, monkeypatch):
+    """The rows of a table past 2^26 go over several launches, here of 128 to
+    1024 rows each: a first launch that only clears the norm pass's slots (9000
+    partials: 141 rows of them) or clears some and updates some, and a last one
+    that ends in padding; three steps, ragged and unaligned tensors, every bit."""
+    monkeypatch.setenv("ARK_OPT_ADAMW_LAUNCH_ROWS", rows)
+    monkeypatch.setenv("ARK_OPT_SUMSQ_SPB", "1")
+    specs = [TensorSpec("a", (4096 * 8990 + 77,), True, False), TensorSpec("b", (257,), False, True),
+             TensorSpec("c", (4096 * 5 + 3,), True, False), TensorSpec("d", (1,), True, False)]
+    cfg, ps, ts, opt, ref = _make(specs, 91, [1e-3] * len(specs), 2048.0, grad_dtype=grad_dtype)
+    for _ in range(3):
+        _, gi = opt.step_all(cfg.lr, info=True)
+        _, ri = ref.step(cfg.lr)
+        assert not H.info_matches(gi, ri)
+    c = H.compare(ps, ts)
+    assert c["w"] == c["m"] == c["v"] == 0, c
+    opt.close()
+
+
 @pytest.mark.parametrize("cap", ["0", "4", "16", "32"])
 def test_adamw_residency_does_not_change_bits(cap, monkeypatch):
     """Any cap on the AdamW waves a CU holds at once (none, the fewest
