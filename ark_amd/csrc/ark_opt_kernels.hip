@@ -989,8 +989,9 @@ int sumsq_spb(uint64_t nseg, uint32_t grad_dtype) {
   // four times the partials to finish (the reading pass gains 4.6 us with 2).
   // Larger blocks only when the partials would exceed kMaxParts (beyond
   // 2^31 elements); 8 covers every table kMaxSegments allows.  A small table
-  // gets smaller blocks until the grid has 2048, the blocks the chip holds at
-  // once: the pass is latency bound until then.  Measured on MI355X, a step
+  // gets smaller blocks until the grid has 2048, about as many as the chip
+  // holds at once (fp16 blocks 1792): latency bound until then, a line set by
+  // measurement.  On MI355X, a step
   // with 1, 2, 4 and 8 segments per block, us: one EKO layer (1729 segments,
   // fp16) 33.0, 34.3, 34.0, 33.2; 2046 segments of fp32 43.1, 44.2, 45.2, 47.1;
   // 5616 segments 90.1, 88.6, 90.5, 92.6 (fp16) and 101.6, 102.0, 103.4, 105.2

@@ -262,8 +262,9 @@ hipError_t launch_adamw_single_w32(float* w, const float* g, float* m, float* v,
 // kFinTarget of (2^19 blocks of 2 segments).
 constexpr uint64_t kClipMaxElements = (uint64_t)kFinTarget * kFoldGroup * 2u * kSeg;
 inline uint32_t clip_parts(uint64_t n) { return (uint32_t)((n + 2u * kSeg - 1) / (2u * kSeg)); }
-// Most blocks of the scaling launch, each of which forms the decision: all of
-// them resident at once.
+// Most blocks of the scaling launch, each of which forms the decision: eight a
+// CU, as many as are resident at once up to 4096 leaves (past them a block's 71
+// registers leave seven).
 constexpr uint64_t kClipBlocks = 2048;
 // parts: clip_parts(n) doubles; folded: ceil(clip_parts(n) / kFoldGroup)
 // doubles (used past kFinTarget partials); norm: device-visible, gets the

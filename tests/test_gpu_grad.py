@@ -42,9 +42,9 @@ def _zipf_tokens(rng, n, vocab, extra=0):
 def test_scatter_matches_oracle(vocab, d, n, extra):
     """Up to 12288 tokens the positions are sorted by counting over 4096-key
     LDS tiles, past that by one hist/scan/scatter launch triple per 8-bit
-    digit over 4096-token tiles: two tiles exactly (8192), a one-token last
-    tile (4097, 12289), one pass (vocab 256), two, and three (vocab 70000 and
-    100000 take 17 key bits)."""
+    digit over 4096-token tiles: two LDS tiles exactly (8192), one key in the
+    last (4097), a one-token last radix tile (12289), one pass (vocab 256) and
+    three (vocab 70000 and 100000 take 17 key bits)."""
     torch = _torch()
     rng = np.random.default_rng(vocab + d + n)
     tokens = _zipf_tokens(rng, n, vocab, extra)
@@ -60,10 +60,10 @@ def test_scatter_matches_oracle(vocab, d, n, extra):
     assert bad.size == 0, f"{len(bad)} elements differ, first {bad[0].tolist()}"
 
 
-def test_scatter_largest_key_ties_with_the_block_sort_padding():
-    """vocab 32768 sorts over 15 bits, where the padding past n (all-ones key)
-    equals the largest real key 32767: the real rows of that token must still
-    come first, in order, and only they are added."""
+def test_scatter_largest_key_in_one_padded_tile():
+    """One LDS tile of the counting sort, padded past n with all-ones keys,
+    many rows of the largest key a 15-bit vocabulary has and one out of range:
+    only the real rows are counted and added, in order."""
     torch = _torch()
     vocab, d, n = 32768, 64, 1000
     rng = np.random.default_rng(13)
@@ -80,13 +80,17 @@ def test_scatter_largest_key_ties_with_the_block_sort_padding():
     np.testing.assert_array_equal(_bits(gg).reshape(vocab, d), want.view(np.uint32))
 
 
-@pytest.mark.parametrize("n", [4097, 8191, 8193])
-def test_scatter_largest_key_ties_with_the_last_tile_padding(n):
-    """Past one tile the last tile's positions beyond n carry the all-ones
-    key too; the real rows of token 32767 (the largest key over 15 bits)
-    spread over every tile must keep their order and land before it."""
+@pytest.mark.parametrize("vocab", [32768, 65536])
+@pytest.mark.parametrize("n", [4097, 8191, 8193, 12287, 12288, 12289, 16383, 16384, 16385])
+def test_scatter_largest_key_ties_with_the_last_tile_padding(n, vocab):
+    """The last tile's positions beyond n carry the all-ones key, in the
+    counting sort (up to 12288 tokens) and in the radix passes past it, where
+    over 15 or 16 bits it equals the largest real key in some or in every
+    digit: the real rows of that key, spread over every tile, must keep their
+    order and land before the padding.  On both sides of where the sorts meet
+    and of a whole radix tile."""
     torch = _torch()
-    vocab, d = 32768, 16
+    d = 16
     rng = np.random.default_rng(n)
     tokens = rng.integers(0, vocab, n).astype(np.uint32)
     tokens[::5] = vocab - 1
@@ -102,15 +106,17 @@ def test_scatter_largest_key_ties_with_the_last_tile_padding(n):
     np.testing.assert_array_equal(_bits(gg).reshape(vocab, d), want.view(np.uint32))
 
 
-def test_scatter_one_long_run_across_tiles():
-    """One token at all 10000 positions: a single run that the multi-tile
-    sort must keep in position order across three tiles, added with the
-    order-revealing values (1e8, 1, -1e8, 1) at the tile seams."""
+@pytest.mark.parametrize("n", [10000, 20000])
+def test_scatter_one_long_run_across_tiles(n):
+    """One token at all positions: a single run that the sort must keep in
+    position order across its 4096-position tiles (10000: counted; 20000: radix
+    passes), added with the order-revealing values (1e8, 1, -1e8, 1) at the tile
+    seams."""
     torch = _torch()
-    vocab, d, n = 50, 64, 10000
+    vocab, d = 50, 64
     rng = np.random.default_rng(17)
     dx0 = rng.standard_normal((n, d)).astype(np.float32)
-    for seam in (4094, 8190):
+    for seam in range(4094, n - 4, 4096):
         dx0[seam:seam + 4, :] = np.array([1e8, 1.0, -1e8, 1.0], np.float32)[:, None]
     tokens = np.full(n, 31, np.uint32)
     want = np.zeros((vocab, d), np.float32)
@@ -140,9 +146,9 @@ def test_scatter_one_long_run_and_order():
 
 @pytest.mark.parametrize("d", [768, 770, 5])
 def test_scatter_run_lengths_at_the_path_boundaries(d):
-    """Runs of 1, 7 and 8 rows (the short and long paths meet at 8) and of
-    59, 60, 61, 120, 121 and 500 rows (the long path adds 60 rows per round,
-    then a tail), positions shuffled, against the oracle."""
+    """Runs of 1, 7 and 8 rows (a wave takes eight at a time below 32 rows)
+    and of 59, 60, 61, 120, 121 and 500 rows (a block's waves take 48 each, the
+    last a remainder), positions shuffled, against the oracle."""
     torch = _torch()
     rng = np.random.default_rng(d)
     lengths = [1, 7, 8, 59, 60, 61, 120, 121, 500]
@@ -337,7 +343,7 @@ def test_scatter_run_lengths_around_the_block_shapes(d, x_off):
 
 @pytest.mark.parametrize("d,g_off", [(768, 0), (4, 0), (68, 0), (100, 0), (1028, 0), (768, 1)])
 def test_scatter_long_runs_at_odd_widths(d, g_off):
-    """Runs of 127 to 1500 rows (many 60-row rounds, then a tail) at widths
+    """Runs of 127 to 1500 rows (many 48-row chunks, then a tail) at widths
     that leave a partial column tile (4, 68, 100, 1028), and with an
     embedding gradient that is only 4-byte aligned (g_off = 1); the
     order-revealing values (1e8, 1, -1e8, 1) straddle rows 510-513 of the

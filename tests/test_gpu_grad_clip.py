@@ -3,7 +3,7 @@ ffi.rs:111-115, :206-220), against the oracle's form of the same call
 (tests/test_oracle_grad_clip.py pins it against the instruction sequence):
 the reported norm and every value after the call bit for bit, clipped and
 not, over sizes from one value to the 24.6M-value embedding gradient and
-past 67M values (the partials folded before the finalize), at unaligned
+past 67M values (the partials folded first), at unaligned
 addresses, with inf, NaN and the compare's edge cases, and queued without
 waiting."""
 import numpy as np
@@ -52,10 +52,21 @@ def test_matches_the_oracle_clipped_and_not(n):
     _check(h, norm * 0.25)  # clipped
 
 
+@pytest.mark.parametrize("parts", [256, 257, 1024, 1025, 4096, 4097, 8192])
+def test_partial_counts_around_the_scaling_blocks_trees(parts):
+    """On both sides of where a lane of the scaling blocks takes 1, 4, 16 or 32
+    partials (256, 1024, 4096 in all) and the most without a fold, the last
+    partial ragged: clipped, and not."""
+    n = parts * 8192 - 5
+    h = np.random.default_rng(parts).standard_normal(n, dtype=F32) * F32(1e-3)
+    norm = _check(h, 1e30)
+    _check(h, norm * 0.5)
+
+
 @pytest.mark.parametrize("n", [67108864 + 1, 70000000])
 def test_past_the_fold_threshold(n):
     """More than 8192 partials (over 67,108,864 values): folded in groups of
-    64 first, as the step folds its own."""
+    64 first."""
     rng = np.random.default_rng(n)
     h = (rng.standard_normal(n) * 1e-3).astype(F32)
     norm = _check(h, 1e30)

@@ -92,19 +92,20 @@ def _pairs(torch, rng, shapes):
     return out
 
 
-# two batches past 4096 tokens (the multi-launch radix sort) whose workspaces
-# fit the 48 MiB array
-_SHAPES = [(32000, 768, 12000), (32000, 512, 16384)]
+# two batches whose workspaces fit the 48 MiB array: one sorted by counting and
+# one by the radix passes, and two by the radix passes
+_SHAPES = [[(32000, 768, 12000), (32000, 512, 16384)], [(32000, 640, 13000), (32000, 512, 16384)]]
 
 
-def test_calls_on_two_streams_take_the_array_in_turn():
+@pytest.mark.parametrize("shapes", _SHAPES)
+def test_calls_on_two_streams_take_the_array_in_turn(shapes):
     """Two different batches queued back to back on two streams, with no
     host wait between them, three times over: each result is the allocating
     call's, bit for bit."""
     torch = _torch()
     L = lib()
     rng = np.random.default_rng(71)
-    cases = _pairs(torch, rng, _SHAPES)
+    cases = _pairs(torch, rng, shapes)
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
     for rep in range(3):
         gots = [g0.clone() for _, _, g0, _ in cases]
@@ -117,13 +118,14 @@ def test_calls_on_two_streams_take_the_array_in_turn():
             assert torch.equal(got.view(torch.int32), want.view(torch.int32)), (rep, k)
 
 
-def test_calls_from_two_host_threads_take_the_array_in_turn():
+@pytest.mark.parametrize("shapes", _SHAPES)
+def test_calls_from_two_host_threads_take_the_array_in_turn(shapes):
     """Two host threads, each with its own stream, each queueing four calls
     into buffers of its own: every result is the allocating call's."""
     torch = _torch()
     L = lib()
     rng = np.random.default_rng(72)
-    cases = _pairs(torch, rng, _SHAPES)
+    cases = _pairs(torch, rng, shapes)
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
     gots = [[g0.clone() for _ in range(4)] for _, _, g0, _ in cases]
     torch.cuda.synchronize()
