@@ -232,10 +232,15 @@ __device__ __forceinline__ double group_tree(double (&q)[R], uint32_t lane) {
 
 // Pairwise tree over the 64 * R partials of one group (0 past nparts) when all
 // have been published; kUnset's value when some have not been after *max_polls
-// more looks at them, and then *max_polls is 0: the wave waits no more.
+// more looks at them, and then *max_polls is 0: the wave waits no more.  more:
+// the wave has several groups after this one, so it looks less often: its looks
+// slow the blocks' stores down (1.3B parameters, norm pass to scalars with sleeps
+// of 1, 4, 10 and 24: 393, 391, 387.5 and 383 us; a table of 7 groups loses
+// 0.5 us when all but the last are looked at seldom).
 template <int R>
 __device__ __forceinline__ double take_group(const double* __restrict__ part, uint32_t nparts,
-                                             uint32_t group, uint32_t lane, uint32_t* max_polls) {
+                                             uint32_t group, uint32_t lane, bool more,
+                                             uint32_t* max_polls) {
   const ARK_GLOBAL uint64_t* p = (const ARK_GLOBAL uint64_t*)part;
   const uint32_t i0 = group * 64u * R + lane;
   uint64_t v[R];
@@ -254,7 +259,10 @@ __device__ __forceinline__ double take_group(const double* __restrict__ part, ui
       *max_polls = 0u;
       return __builtin_bit_cast(double, kUnset);
     }
-    __builtin_amdgcn_s_sleep(1);
+    if (more)
+      __builtin_amdgcn_s_sleep(24);
+    else
+      __builtin_amdgcn_s_sleep(1);
   }
   double q[R];
 #pragma unroll
@@ -275,7 +283,8 @@ __device__ __forceinline__ double take_all(const double* __restrict__ part, uint
   for (uint32_t i = threadIdx.x; i < kFinGroups; i += kBlock)
     if (i >= groups) sums[i] = 0.0;
   for (uint32_t k = wave; k < groups; k += kBlock / 64) {
-    const double x = take_group<R>(part, nparts, groups - 1u - k, lane, &max_polls);
+    const double x = take_group<R>(part, nparts, groups - 1u - k, lane,
+                                   k + 4u * (kBlock / 64) < groups, &max_polls);
     if (lane == 0) sums[groups - 1u - k] = x;
   }
   __syncthreads();

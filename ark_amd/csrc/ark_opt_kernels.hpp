@@ -118,7 +118,7 @@ constexpr uint32_t kMaxParts = kFinGroups * 64u * 8u;
 
 // How often a finalizer wave looks for the partials of one group (1024 at
 // most) before it gives the step up: each look is a round trip past the L2s and
-// a sleep, 0.7 to 1 us together on MI355X, so the wait lasts over ten seconds.
+// a sleep, 0.7 us or more together on MI355X, so the wait lasts over ten seconds.
 // The norm pass of 1.2B parameters takes at most 13 looks at a group; what the
 // bound leaves room for is other work on the GPU that holds the pass back.
 constexpr uint32_t kFinMaxPolls = 1u << 24;
