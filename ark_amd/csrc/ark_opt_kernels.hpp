@@ -190,31 +190,36 @@ uint32_t sumsq_lds_for(uint32_t grad_dtype, int spb, int blocks);
 // dynamic-LDS reservation: more waves hide the latency of what the norm pass
 // left in the Infinity Cache, but over-issue the seven streams that come from
 // HBM, so the fewer the larger the uncached share; a step from units finds
-// nothing cached.  Measured on MI355X, step in us (two tables in turn, 15
-// rounds in a random order; the rounds' 10th and 90th percentiles lie within
-// 0.2 % of the median):
+// nothing cached.  Measured on MI355X, step in us over tables taken in turn, as
+// many as are together past 1 GB (the cache holds 256 MB, and a trainer's forward
+// and backward come between steps); 15 rounds in a random order, whose 10th and
+// 90th percentiles lie within 0.2 % of the median:
 //   waves                     12       16       20       24
-//   fp16 gradients     7M     33.86    32.93    33.69    33.05
-//                      20M    80.63    78.90    78.66    78.26
-//                      45M   164.9    160.8    161.4    162.1
-//                      90M   325.2    314.7    315.2    318.1
-//                      131M  469.3    457.1    457.3    461.9
+//   fp16 gradients     3M     19.25    18.90    19.30    18.60
+//                      7M     33.75    32.90    33.28    32.56
+//                      20M    79.51    77.61    77.66    76.95
+//                      33M   125.2    121.4    121.3    121.0
+//                      45M   163.9    158.7    160.0    159.7
+//                      90M   323.1    309.9    309.8    312.3
+//                      131M  468.3    453.2    454.7    458.0
 //                      237M  849.7    829.0    832.6    840.1
-//   fp32 gradients     8M     40.14    39.66    39.06    38.81
-//                      20M    90.57    88.02    87.34    87.43
-//                      45M   192.4    187.7    185.7    186.0
-//                      90M   379.9    375.1    373.4    375.4
-//                      131M  550.1    547.7    547.1    550.0
-//                      270M 1149.8   1151.5   1151.4   1158.7
+//   fp32 gradients     3M     20.55    20.44    20.17    19.52
+//                      8M     44.63    43.59    42.97    42.95
+//                      20M    91.14    88.84    87.75    88.39
+//                      45M   191.8    189.4    186.3    187.3
+//                      90M   377.7    372.3    369.6    371.4
+//                      131M  549.5    547.0    545.9    547.9
+//                      180M  763.9    767.9    765.7    770.6
 //                      404M 1718.5   1722.2   1722.6   1729.8
 //                      640M 2713.6   2740.5   2746.2   2762.2
-//   from units         10M    62.77    62.96    62.65    62.60
-//   (with the          45M   254.5    255.8    256.0    256.7
-//   accumulation)      237M 1280.9   1291.5   1300.4   1303.3
+//   from units         3M     25.97    25.84    25.57    25.53
+//   (with the          10M    64.65    64.73    64.25    64.37
+//   accumulation)      45M   253.2    253.5    253.9    254.6
+//                      237M 1280.9   1291.5   1300.4   1303.3
 inline int adamw_waves(uint64_t nseg, uint32_t grad_dtype, bool from_units) {
-  if (grad_dtype == ARK_OPT_GRAD_F16) return 16;
-  if (from_units || nseg > (1u << 15)) return 12;  // 134M parameters
-  return nseg <= (1u << 12) ? 24 : 20;             // 17M
+  if (from_units) return 12;
+  if (grad_dtype == ARK_OPT_GRAD_F16) return nseg <= (1u << 13) ? 24 : 16;    // 34M parameters
+  return nseg <= (1u << 12) ? 24 : nseg <= (1u << 15) ? 20 : 12;             // 17M, 134M
 }
 // The dynamic LDS that holds the AdamW kernel for grad_dtype at `waves` per
 // CU, rounded up to whole blocks (resident_lds_bytes; 0 = no cap).
