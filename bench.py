@@ -149,7 +149,7 @@ def _run_gpu(name, steps, warmup, stream, grad="f16", skip=False):
     res = dict(skip=skip,
         n_params=n, n_tensors=len(specs), ms_step=ms_step,
         ms_adamw=tm.ms_adamw / tm.steps, ms_norm=tm.ms_norm / tm.steps,
-        ms_finalize=tm.ms_finalize / tm.steps, ms_step_events=tm.ms_step / tm.steps,
+        ms_step_events=tm.ms_step / tm.steps,
         clipped=int(last.clipped), applied=int(last.applied), t=int(last.state.t),
         grad_norm=float(last.grad_norm), graph_ms=graph_ms,
     )
@@ -161,10 +161,9 @@ def _run_gpu(name, steps, warmup, stream, grad="f16", skip=False):
 
 def _time_skipped(ps, opt, cfg, steps):
     """steps skipped steps (training.rs:293-305): +inf planted in one fp16
-    gradient, so the norm pass flags it, the finalize halves the loss scale
-    and counts the skip, and the AdamW pass exits at once.  Wall clock over
-    the steps, and the kernels with the handle's events; the gradient is
-    restored afterwards."""
+    gradient, so the norm pass flags it, halves the loss scale and counts the
+    skip, and the AdamW pass exits at once.  Wall clock over the steps, and the
+    norm pass with the handle's events; the gradient is restored afterwards."""
     import torch
     g16 = ps.g(0).view(torch.int16)
     old = int(g16[0].item())
@@ -186,14 +185,12 @@ def _time_skipped(ps, opt, cfg, steps):
     _, last = opt.step_all(cfg.lr, info=True)
     g16[0] = old
     assert last.applied == 0 and last.state.skipped_steps >= 2 * steps + 2
-    log(f"[bench] skipped step: {wall_ms:.4f} ms (norm {tm.ms_norm / tm.steps:.4f}, finalize "
-        f"{tm.ms_finalize / tm.steps:.4f})")
+    log(f"[bench] skipped step: {wall_ms:.4f} ms (norm {tm.ms_norm / tm.steps:.4f})")
     # the AdamW launch's own event interval is left out: events around a
     # launch whose blocks all exit at once read longer than the whole
     # skipped step's wall clock; rocprofv3's kernel trace times that dispatch
     return dict(ms_per_skipped_step=round(wall_ms, 4),
-                kernels_ms={"sumsq": round(tm.ms_norm / tm.steps, 4),
-                            "finalize": round(tm.ms_finalize / tm.steps, 4)},
+                kernels_ms={"sumsq": round(tm.ms_norm / tm.steps, 4)},
                 skipped_total=int(last.state.skipped_steps))
 
 
@@ -266,7 +263,7 @@ def _run_fused(specs, ps, opt, cfg, steps, warmup, stream):
     res = dict(
         n_params=ps.n_params, n_tensors=n, ms_step=step_fused,
         ms_adamw=tf.ms_adamw / tf.steps, ms_norm=tf.ms_norm / tf.steps,
-        ms_finalize=tf.ms_finalize / tf.steps, ms_step_events=tf.ms_step / tf.steps,
+        ms_step_events=tf.ms_step / tf.steps,
         clipped=int(last.clipped), applied=int(last.applied), t=int(last.state.t),
         grad_norm=float(last.grad_norm), graph_ms=None,
         fused=dict(producer_ms=round(producer_ms, 4), pair_ms=round(pair_fused, 4),
@@ -457,8 +454,7 @@ def secondary_c4(steps, warmup):
                frac_of_peak_hbm=round(gbs / PEAK_HBM_GBS, 4),
                bytes_per_step=b_step * n, clipped=r["clipped"],
                hip_graph_ms_per_step=round(r["graph_ms"], 4),
-               kernels_ms={"sumsq": round(r["ms_norm"], 4), "finalize": round(r["ms_finalize"], 4),
-                           "adamw": round(r["ms_adamw"], 4)},
+               kernels_ms={"sumsq": round(r["ms_norm"], 4), "adamw": round(r["ms_adamw"], 4)},
                adamw=dict(achieved=round(adam_gbs, 2), unit="GB/s",
                           frac=round(adam_gbs / PEAK_HBM_GBS, 4),
                           algorithmic_bytes_per_launch=b_adamw * n))
@@ -1002,8 +998,8 @@ def main():
                                       else None),
         },
         "frac_of_peak_hbm": round(gbs / PEAK_HBM_GBS, 4),
-        "kernels_ms": {"sumsq": round(r["ms_norm"], 4), "finalize": round(r["ms_finalize"], 4),
-                       "adamw": round(r["ms_adamw"], 4), "step_events": round(r["ms_step_events"], 4)},
+        "kernels_ms": {"sumsq": round(r["ms_norm"], 4), "adamw": round(r["ms_adamw"], 4),
+                       "step_events": round(r["ms_step_events"], 4)},
         "roofline": {
             "kernel": "adamw_kernel",
             "bound": "hbm",
@@ -1022,18 +1018,17 @@ def main():
             "c3_skipped_step": dict(
                 r["skip"], workload="c3: the c2 set with +inf in one fp16 gradient",
                 bytes_per_skipped_step=2 * n,
-                note="the norm pass reads g (2 B/param) and flags it, the finalize skips and "
-                     "halves the loss scale, the AdamW pass exits before any access; the rest "
-                     "of the wall clock is that exiting launch's dispatch (kernel trace: "
-                     "profiles/adamw_kernel_c3.md)"),
+                note="the norm pass reads g (2 B/param), flags it and halves the loss scale, "
+                     "the AdamW pass exits before any access; the rest of the wall clock is "
+                     "that exiting launch (kernel trace: profiles/adamw_kernel_c3.md)"),
             "c4": c4,
         }
     elif r.get("skip"):
         out["config"]["skipped_steps"] = dict(
             r["skip"], ms_per_applied_step=round(r["ms_step"], 4),
             bytes_per_skipped_step=2 * n,
-            note="an inf in one gradient: the norm pass reads g (2 B/param) and flags it, the "
-            "finalize skips, the AdamW pass exits before any access")
+            note="an inf in one gradient: the norm pass reads g (2 B/param), flags it and "
+            "halves the loss scale, the AdamW pass exits before any access")
     if a.grad == "f32-fused":
         out["config"]["fused_norm"] = dict(
             r["fused"], note="ms_per_step: the step after the gradient plan's final "

@@ -128,9 +128,10 @@ typedef struct ark_opt_step_info {
 /* Per-kernel device time accumulated while timing is enabled. */
 typedef struct ark_opt_timing {
   uint64_t steps;     /* steps timed                                   */
-  double ms_norm;     /* total ms in the sum-of-squares / finite kernel */
-  double ms_finalize; /* total ms from there to the AdamW pass (the norm
-                       * pass also finishes the step's scalars)         */
+  double ms_norm;     /* total ms in the norm pass, scalars included    */
+  double ms_finalize; /* total ms between two events recorded one after
+                       * the other between the passes: their own cost, no
+                       * kernel (the norm pass finishes the scalars)    */
   double ms_adamw;    /* total ms in the fused AdamW kernel             */
   double ms_step;     /* total ms from the first to the last kernel     */
 } ark_opt_timing;
