@@ -815,9 +815,11 @@ ScatterLayout scatter_layout(uint32_t n) {
   return L;
 }
 
-// What the no-allocation call counts a batch as against its static array (the
-// size stated in include/ark_grad.h, which also allows for a copy of dx0):
-// never less than scatter_layout takes.
+// What the no-allocation call counts a batch as against its static array: the
+// size stated in include/ark_grad.h, which allows for a copy of dx0 that the
+// kernels no longer make.  Kept, so that which batches the call takes is a
+// matter of the interface and not of the sort behind it; never less than
+// scatter_layout takes.
 size_t noalloc_need(uint32_t n, uint32_t d) {
   const size_t arr = ark::align_up((size_t)n * 4, 256);
   size_t need = 2 * arr + ark::align_up((size_t)n * d * 4, 256);

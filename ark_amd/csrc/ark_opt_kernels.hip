@@ -201,12 +201,12 @@ constexpr int log2i(int v) { return v <= 1 ? 0 : 1 + log2i(v / 2); }
 // step's AdamW pass put kUnset back, so every pass starts from clear slots.  The
 // wait is bounded (FinalizeArgs::max_polls): where two runs of one handle
 // overlap, one's AdamW pass may clear partials the other's finalizer waits for,
-// whose step then ends with nothing updated.  What it costs is the time from the last
-// partial to the scalars.  Measured on MI355X, norm pass to scalars, us (a norm
-// kernel, past 8192 partials a fold, and a one-block finalize before): one
-// 768 x 768 tensor 4.8 (3.2 + 3.3 and a launch between), one layer 7.8 (5.7 +
-// 4.0), EKO-237M 76.4 (73.3 + 4.7 + 4.6), from units 7.8 (4.8 + 4.8), the 1.3B
-// set 373 (373 + 5 + 5).
+// whose step then ends with nothing updated.  What it costs is the time from the
+// last partial to the scalars.  Measured on MI355X, norm pass to scalars, us (a
+// norm kernel, past 8192 partials a fold, and a one-block finalize, with launches
+// between, before): one 768 x 768 tensor 4.8 (3.2 + 3.3), one layer 7.8 (5.7 +
+// 4.0), EKO-237M 75.4 (72.4 + 4.5 + 4.3), from units 8.0 (4.8 + 4.8), the 1.3B
+// set 389 (367 + 4.6 + 4.3).
 
 constexpr uint64_t kUnset = ~0ull;  // a NaN that publish() never stores
 
@@ -437,8 +437,9 @@ __device__ __forceinline__ void fast_batch(const SegDesc (&dsc)[kRed], int tid, 
 
 // Block 0 is the finalizer.  The others cover segments [b*SPB, b*SPB + SPB)
 // (SPB <= 8) each, b counted from the last, and publish the pairwise tree of
-// their 2*SPB half-segment sums: an aligned subtree of the global tree.  A block that saw an inf or NaN gradient writes NaN, so the
-// global sum is NaN exactly when some gradient is non-finite (training.rs:291).
+// their 2*SPB half-segment sums: an aligned subtree of the global tree.  A block
+// that saw an inf or NaN gradient writes NaN, so the global sum is NaN exactly when
+// some gradient is non-finite (training.rs:291).
 // Blocks from nt_from up read with non-temporal loads: they run first, and
 // what they read would leave the Infinity Cache before the AdamW pass gets
 // there; the blocks below (the last ~256 MiB read, where AdamW starts) keep
@@ -623,7 +624,7 @@ __global__ void record_overflow_kernel(ark_opt_hparams hp,
   if (host_info) *host_info = out;
 }
 
-// ---- kernel 3: fused AdamW -------------------------------------------------
+// ---- kernel 2: fused AdamW -------------------------------------------------
 
 struct ElemConsts {
   float beta1, beta2, c1, c2, eps, lr_eff, decay;
@@ -718,11 +719,11 @@ __device__ __forceinline__ void adam_row(uint16_t* w, const GT* g, float* m, flo
 // kAdamStride of the blocks' group b / kAdamStride: neighbouring rows run at the
 // same time on neighbouring blocks, hence on different XCDs, as with one row
 // per block, while a block dispatches kAdamWaves waves at once.  HBM bound;
-// what a skipped step pays is the dispatch.  Measured on MI355X, EKO-237M
-// (step / skipped step, us): one-wave blocks 842 / 287; blocks of two waves on
-// adjacent rows 877 / 191, on rows 64 apart 845 / 191; four waves 32 rows apart
-// 838 / 175, 16 apart 847, 64 apart 843, 128 apart 854; eight waves 852 / 181;
-// two rows per wave 850 / 155-190, four 872 / 140-160.
+// what a skipped step pays is the dispatch and each wave's one load.  Measured on
+// MI355X, EKO-237M (step / skipped step, us): one-wave blocks 842 / 287; blocks of
+// two waves on adjacent rows 877 / 191, on rows 64 apart 845 / 191; four waves 32
+// rows apart 838 / 175, 16 apart 847, 64 apart 843, 128 apart 854; eight waves
+// 852 / 181; two rows per wave 850 / 155-190, four 872 / 140-160.
 // The rows below `first` are the norm pass's slots (slot_rows).  They are the
 // first, and a branch the compiler leaves out of line, because a leaving wave
 // costs what its few scalar instructions do (skipped step's pass, us: 80.9 both
