@@ -188,38 +188,40 @@ constexpr int kSumsqBlocksPerCuF16 = 7;
 uint32_t sumsq_lds_for(uint32_t grad_dtype, int spb, int blocks);
 // Resident AdamW waves per CU for a table of nseg segments, held by a
 // dynamic-LDS reservation: more waves hide the latency of what the norm pass
-// left in the Infinity Cache, but over-issue the seven streams that come from
-// HBM, so the fewer the larger the uncached share; a step from units finds
-// nothing cached.  Measured on MI355X, step in us over tables taken in turn, as
-// many as are together past 1 GB (the cache holds 256 MB, and a trainer's forward
-// and backward come between steps); 15 rounds in a random order, whose 10th and
-// 90th percentiles lie within 0.2 % of the median:
-//   waves                     12       16       20       24
-//   fp16 gradients     3M     19.25    18.90    19.30    18.60
-//                      7M     33.75    32.90    33.28    32.56
-//                      20M    79.51    77.61    77.66    76.95
-//                      33M   125.2    121.4    121.3    121.0
-//                      45M   163.9    158.7    160.0    159.7
-//                      90M   323.1    309.9    309.8    312.3
-//                      131M  468.3    453.2    454.7    458.0
-//                      237M  849.7    829.0    832.6    840.1
-//   fp32 gradients     3M     20.55    20.44    20.17    19.52
-//                      8M     44.63    43.59    42.97    42.95
-//                      20M    91.14    88.84    87.75    88.39
-//                      45M   191.8    189.4    186.3    187.3
-//                      90M   377.7    372.3    369.6    371.4
-//                      131M  549.5    547.0    545.9    547.9
-//                      180M  763.9    767.9    765.7    770.6
-//                      404M 1718.5   1722.2   1722.6   1729.8
-//                      640M 2713.6   2740.5   2746.2   2762.2
-//   from units         3M     25.97    25.84    25.57    25.53
-//   (with the          10M    64.65    64.73    64.25    64.37
-//   accumulation)      45M   253.2    253.5    253.9    254.6
+// left in the Infinity Cache and of a skipped step's one load, but over-issue
+// the seven streams that come from HBM, so the fewer the larger the uncached
+// share; a step from units finds nothing cached.  Measured on MI355X over
+// models' tables, step in us (two to five tables in turn, 9 rounds in a random
+// order, whose 10th and 90th percentiles lie within 0.4 % of the median; a
+// skipped step behind the bar):
+//   waves                     12       16       20       24   |  12   16   20   24
+//   fp16 gradients     7M     33.74    33.08    33.36    32.62
+//                      21M    85.0     83.2     82.8     81.6
+//                      39M   147.5    141.6    141.4    141.0 |  35   32   30   29
+//                      60M   223.9    215.3    214.9    215.2 |  49   45   42   40
+//                      82M   303.1    291.1    291.8    289.6 |  68   62   58   56
+//                      110M  395.1    378.1    379.2    378.4 |  85   77   72   69
+//                      159M  579.3    570.1    576.7    579.7 | 120  109  101   97
+//                      237M  862.6    840.5    843.5    846.3 | 173  156  144  138
+//                      334M 1232.0   1219.5   1240.8   1249.5 | 245  219  202  194
+//   fp32 gradients     7M     37.00    36.34    35.64    35.78
+//                      21M    96.6     94.0     92.3     91.8
+//                      39M   171.6    166.0    164.1    162.7
+//                      82M   355.3    347.7    345.6    343.8
+//                      110M  468.5    460.4    458.1    458.2
+//                      159M  692.4    694.5    697.7    697.4
+//                      180M  782.7    776.5    778.1    783.3
+//                      237M 1015.9   1013.5   1009.3   1009.8
+//                      273M 1192.5   1204.0   1209.6   1213.8
+//                      334M 1464.4   1478.1   1488.0   1491.1
+//   from units         10M    64.65    64.73    64.25    64.37  (with the
+//                      45M   253.2    253.5    253.9    254.6   accumulation)
 //                      237M 1280.9   1291.5   1300.4   1303.3
 inline int adamw_waves(uint64_t nseg, uint32_t grad_dtype, bool from_units) {
   if (from_units) return 12;
-  if (grad_dtype == ARK_OPT_GRAD_F16) return nseg <= (1u << 13) ? 24 : 16;    // 34M parameters
-  return nseg <= (1u << 12) ? 24 : nseg <= (1u << 15) ? 20 : 12;             // 17M, 134M
+  if (nseg <= (1u << 15)) return 24;  // 134M parameters
+  if (grad_dtype == ARK_OPT_GRAD_F16) return 16;
+  return nseg <= (1u << 16) ? 20 : 12;  // 268M
 }
 // The dynamic LDS that holds the AdamW kernel for grad_dtype at `waves` per
 // CU, rounded up to whole blocks (resident_lds_bytes; 0 = no cap).
